@@ -210,9 +210,8 @@ int mfd_mode_attn(const uint16_t* q, int64_t q_st, int64_t q_sh, const uint16_t*
  * lane / wave order, piece terms combined in fp64), exactly reproducible on the CPU.
  * k = 0: log Z only. Rows must start 16-byte aligned (row_stride % 8 == 0), and the buffer must hold
  * rows * row_stride elements (the last row's tail is read in 16-byte units up to the next multiple of 8).
- * Requires k <= 256 and a row merge of at most 8192 candidates: ceil(V / 2048) * max(k, 1) <= 8192 for
- * k <= 32 (one candidate list per 2048-element piece), ceil(V / 8192) * k <= 8192 for k > 32 (one list per
- * 8192 elements); beyond that MFD_ERR_UNSUPPORTED. mfd_topk_logz_workspace_bytes(rows, V, k) =
+ * Requires k <= 256, and ceil(V / 2048) * max(k, 1) <= 8192 for k <= 32, ceil(V / 8192) * k <= 8192 for
+ * k > 32; beyond that MFD_ERR_UNSUPPORTED. mfd_topk_logz_workspace_bytes(rows, V, k) =
  * rows * ceil(V / 2048) * (12 + 8 max(k, 1)) + 64 bytes.
  */
 int64_t mfd_topk_logz_workspace_bytes(int rows, int V, int k);

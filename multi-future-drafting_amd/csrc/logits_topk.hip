@@ -15,20 +15,14 @@
 //   Z = sum_c S_c exp_det(max(m_c - m, -80)) in piece order (fp64), log Z = float(m + log_det(Z)).
 // exp_det and log_det use only IEEE +, *, fma, division and exact power-of-two scaling, with contraction
 // disabled; log Z agrees with an fp64 logsumexp to about one fp32 ulp.
-// The table index of a bf16 bit pattern b is min(max(rotl16(b, 1) - 0x6600, 0), 8191), formed for two
-// elements at once with packed 16-bit operations; the table sits in LDS (32 KB, staged once per workgroup
-// with direct-to-LDS loads).
 //
-// Kernel 1 (k <= 32): one wave per piece, no workgroup barrier after the table: the piece's maximum, its sum
-//           S_c and its top k (the k-th largest 16-bit value key of the 64 lane maxima is a threshold that the
-//           piece's top k all reach; only the 8-element groups whose maximum reaches it are listed, and only
-//           their elements get order keys, which are ranked by counting); the k keys are written in rank order.
-// Kernel 1 (k > 32): one workgroup of four waves per 8192 elements (four pieces): the pieces' sums as above,
-//           and the top k of the 8192 elements (per-thread sorted lists, merged per wave, then per block).
-// Kernel 2: one wave per row: combines the piece sums and merges the sorted candidate lists, writes
-//           log-probs / ids.
+// Kernel 1 (topk_piece_kernel): one wave per piece: its maximum, its sum S_c, and the largest key of each of its 16
+//           groups of 128 elements. No selection and no synchronisation between waves.
+// Kernel 2 (topk_row_kernel): one workgroup per row: the k-th largest group maximum t; at least k elements reach t,
+//           and all that do lie in the few groups whose maximum does, which are read again (from the caches): their
+//           elements from t up are the candidates, whose exact top k it takes. Log Z and the outputs.
+// A row of at most 16 pieces is done by one workgroup in one launch.
 #include <algorithm>
-#include <atomic>
 
 #include "mfd_common.h"
 #include "exp_bf16_table.h"
@@ -38,11 +32,10 @@
 namespace {
 
 constexpr int PIECE = MFD_LZ_PIECE;  // log Z piece: one wave, 32 elements per lane
-constexpr int CHUNK = 4 * PIECE;     // top-k unit of the k > 32 kernel (one workgroup of four waves)
-constexpr int NT = 256;
-constexpr int PER = CHUNK / NT;      // 32 elements per thread
-constexpr int FINAL_STAGE = 4096;    // candidates per row staged in LDS by the k <= 32 merge (32 KB)
-constexpr int KMAX = 256;            // a thread holds 32 elements: its 32-entry list keeps all of them for k > 32
+constexpr int PW = 16;               // waves per workgroup of kernel 1
+constexpr int NT1 = PW * 64;
+constexpr int KMAX = 256;
+constexpr int MERGE_MAX = 8192;      // accepted sizes: pieces * k (k <= 32), ceil(V / 8192) * k above
 
 __device__ __forceinline__ float pow2i(int k) { return __uint_as_float((uint32_t)(k + 127) << 23); }
 
@@ -89,68 +82,75 @@ __device__ double log_det(double z) {
   const double de = (double)e;
   return __builtin_fma(de, 6.93147180369123816490e-01, __builtin_fma(de, 1.90821492927058770002e-10, logf_));
 }
-
 // ---- the e^x table ------------------------------------------------------------------------------------
+// In LDS the 8192 entries are split by sign: e^x of the non-negative magnitudes i at byte 4 i, of the negative
+// ones at byte 32768 + 4 i, so that the byte offset of a bf16 bit pattern b is
+//   4 min(max((b & 0x7FFF) - 0x3300, 0), 4095) + (b & 0x8000),
+// five packed 16-bit operations for two elements. Entry 4095 of the non-negative half (x = 127.5, and every
+// larger magnitude and NaN) holds 0: no element of a piece with m_c < 64 is that large, and a NaN adds nothing.
 constexpr int ETAB = MFD_EXP_BF16_TABLE_SIZE;
+constexpr int ETAB_NEG = 32768;              // byte offset of the negative half; the 16 KB in between are free
+constexpr int ETAB_BYTES = ETAB_NEG + ETAB * 2;
 __device__ const uint32_t exp_tab_g[ETAB] = {MFD_EXP_BF16_TABLE_INIT};
 typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
+typedef int16_t i16x2 __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef uint64_t u64x2 __attribute__((ext_vector_type(2)));
 
-// Byte offsets (4 idx) into the table of the two bf16 values of a packed pair, in the two 16-bit halves:
-// idx = min(max(rotl16(b, 1) - 0x6600, 0), 8191); v_pk_lshlrev_b16 / v_pk_lshrrev_b16 / v_pk_sub_u16 clamp /
-// v_pk_min_u16, six operations for two elements.
 __device__ __forceinline__ uint32_t etab_offsets(uint32_t pair) {
   const u16x2 b = __builtin_bit_cast(u16x2, pair);
-  const u16x2 r = (b << (u16x2){1, 1}) | (b >> (u16x2){15, 15});
-  u16x2 i = __builtin_elementwise_sub_sat(r, (u16x2){0x6600, 0x6600});
-  i = __builtin_elementwise_min(i, (u16x2){ETAB - 1, ETAB - 1});
-  return __builtin_bit_cast(uint32_t, (u16x2)(i << (u16x2){2, 2}));
+  u16x2 i = __builtin_elementwise_sub_sat((u16x2)(b << (u16x2){1, 1}), (u16x2){0x6600, 0x6600});
+  i = __builtin_elementwise_min(i, (u16x2){ETAB - 2, ETAB - 2});
+  // (pair & 0x80008000) | 2 i in one operation (the compiler takes it apart into three)
+  uint32_t off;
+  asm("v_and_or_b32 %0, %1, %2, %3"
+      : "=v"(off)
+      : "v"(pair), "s"(0x80008000u), "v"(__builtin_bit_cast(uint32_t, (u16x2)(i << (u16x2){1, 1}))));
+  return off;
 }
-__device__ __forceinline__ float etab_at(const float* etab, uint32_t byte_off) {
-  return *reinterpret_cast<const float*>(reinterpret_cast<const char*>(etab) + byte_off);
+__device__ __forceinline__ float etab_at(const unsigned char* etab, uint32_t byte_off) {
+  return *reinterpret_cast<const float*>(etab + byte_off);
 }
-
-// One direct-to-LDS load (global_load_lds_dwordx4): lane l's 16 bytes at base + off land at LDS byte address
-// lds_byte + 16 l (base and lds_byte wave-uniform). Waited for with s_waitcnt vmcnt(0) before the barrier that
-// publishes the table.
-__device__ __forceinline__ void dma16(const void* base, uint32_t off, uint32_t lds_byte) {
-  const uint32_t l = __builtin_amdgcn_readfirstlane(lds_byte);
-  const uint64_t bb = (uint64_t)(uintptr_t)base;
-  const uint64_t bs = ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(bb >> 32)) << 32) |
-                      (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)bb);
-  asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(l), "v"(off), "s"(bs) : "memory", "m0");
-}
-// The table into LDS by the nwaves waves of a workgroup, 1 KB per load.
-__device__ __forceinline__ void etab_stage(float* etab, int nwaves) {
-  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) float*)etab;
-  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  for (int piece = w; piece < ETAB * 4 / 1024; piece += nwaves) {
-    const uint32_t off = (uint32_t)piece * 1024u;
-    dma16(exp_tab_g, off + 16u * lane, lds0 + off);
-  }
+// The table into LDS by all NT1 threads: entries 8 t .. 8 t + 7 (magnitudes 4 t .. 4 t + 3, both signs).
+__device__ __forceinline__ void etab_stage(unsigned char* etab) {
+  static_assert(ETAB == 8 * NT1, "eight entries per thread");
+  const int t = threadIdx.x;
+  const u32x4 a = reinterpret_cast<const u32x4*>(exp_tab_g)[2 * t];
+  const u32x4 b = reinterpret_cast<const u32x4*>(exp_tab_g)[2 * t + 1];
+  *reinterpret_cast<u32x4*>(etab + 16 * t) = (u32x4){a[0], a[2], b[0], t == NT1 - 1 ? 0u : b[2]};
+  *reinterpret_cast<u32x4*>(etab + ETAB_NEG + 16 * t) = (u32x4){a[1], a[3], b[1], b[3]};
 }
 
 // Lane sum of one piece: the lane's 32 elements raw[j][e] (piece element 512 j + 8 lane + e) in (j, e) order,
-// against the piece maximum m. Elements at piece positions >= nvalid are past the row end: -inf in raw,
+// against the piece maximum m. Elements at piece positions >= nvalid are past the row end: NaNs in raw,
 // contributing nothing. The polynomial path (m outside the table's range, rare) reads the elements again
 // from psrc, the piece's first element.
-__device__ __forceinline__ float piece_lane_sum(const u16x8 (&raw)[4], float m, const uint16_t* psrc, int nvalid,
-                                                const float* etab) {
+__device__ __forceinline__ float piece_lane_sum(const u32x4 (&raw)[4], float m, const uint16_t* psrc, int nvalid,
+                                                const unsigned char* etab) {
 #pragma clang fp contract(off)
   float s = 0.f;
   if (m >= -60.0f && m < 64.0f) {
     // -m is a bf16 value too: its bits are m's upper half with the sign flipped
     const uint32_t mneg = ((__float_as_uint(m) >> 16) ^ 0x8000u) * 0x10001u;
     const float C = etab_at(etab, etab_offsets(mneg) & 0xFFFFu);
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const u32x4 u = __builtin_bit_cast(u32x4, raw[j]);
+    // the eight table reads of group j + 1 are in flight while those of group j are added (left to itself the compiler
+    // waits for every read before the next)
+    float x[2][8];
+    auto fetch = [&](int j) {
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
-        const uint32_t off = etab_offsets(u[q]);
-        s = __builtin_fmaf(etab_at(etab, off & 0xFFFFu), C, s);
-        s = __builtin_fmaf(etab_at(etab, off >> 16), C, s);
+        const uint32_t off = etab_offsets(raw[j][q]);
+        x[j & 1][2 * q] = etab_at(etab, off & 0xFFFFu);
+        x[j & 1][2 * q + 1] = etab_at(etab, off >> 16);
       }
+    };
+    fetch(0);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      if (j < 3) fetch(j + 1);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) s = __builtin_fmaf(x[j & 1][e], C, s);
     }
   } else if (m != -INFINITY) {
     const int l8 = 8 * (int)(threadIdx.x & 63);
@@ -171,56 +171,29 @@ __device__ __forceinline__ float piece_lane_sum(const u16x8 (&raw)[4], float m, 
   return s;
 }
 
-// Sum over the wave, pairwise over lane distances 32, 16, 8, 4, 2, 1: every lane ends with the same value.
-__device__ __forceinline__ float wave_sum_tree(float v) {
-#pragma clang fp contract(off)
-  const int lane = threadIdx.x & 63;
-#pragma unroll
-  for (int d = 32; d >= 1; d >>= 1)
-    v = v + __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute((lane ^ d) << 2, __builtin_bit_cast(int, v)));
-  return v;
-}
-
-// ---- keys and wave reductions -------------------------------------------------------------------------
-// candidate key: larger = better (value descending, then token id ascending)
-__device__ __forceinline__ uint64_t cand_key(float x, uint32_t idx) {
-  return ((uint64_t)float_order_key(x + 0.0f) << 32) | (uint64_t)(0xFFFFFFFFu - idx);
-}
-
-__device__ __forceinline__ uint64_t shfl_xor_u64(uint64_t v, int mask) {
-  const int lane = threadIdx.x & 63;
-  const int src = (lane ^ mask) << 2;
-  const uint32_t lo = (uint32_t)__builtin_amdgcn_ds_bpermute(src, (int)(uint32_t)v);
-  const uint32_t hi = (uint32_t)__builtin_amdgcn_ds_bpermute(src, (int)(uint32_t)(v >> 32));
-  return ((uint64_t)hi << 32) | lo;
-}
-__device__ __forceinline__ uint64_t wave_max_u64(uint64_t v) {
-#pragma unroll
-  for (int m = 32; m >= 1; m >>= 1) {
-    const uint64_t o = shfl_xor_u64(v, m);
-    v = o > v ? o : v;
-  }
-  return v;
-}
-
-// one list per thread, merged across the wave: k rounds of "best head wins"
-template <int KT>
-__device__ void wave_topk(const uint64_t (&list)[KT], int k, uint64_t* out /* LDS, k entries */) {
-  int head = 0;
-  for (int i = 0; i < k; ++i) {
-    uint64_t mine = 0;
-#pragma unroll
-    for (int j = 0; j < KT; ++j)
-      if (j == head) mine = list[j];
-    const uint64_t best = wave_max_u64(mine);
-    if (best != 0 && mine == best) ++head;  // keys are unique (they contain the token id)
-    if ((threadIdx.x & 63) == 0) out[i] = best;
-  }
-}
-
+// ---- wave reductions ------------------------------------------------------------------------------------
 template <int N>
 __device__ __forceinline__ uint32_t row_ror32(uint32_t v) {
   return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x120 + N, 0xF, 0xF, false);
+}
+// Sum over the wave, pairwise over lane distances 32, 16, 8, 4, 2, 1: every lane ends with the same value. Once
+// the distances above d are added, a lane's value depends only on its number modulo 2 d, so a rotation by d
+// within the row of 16 reads the same value as lane ^ d.
+__device__ __forceinline__ float wave_sum_tree(float v) {
+#pragma clang fp contract(off)
+  {
+    const auto p = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = __uint_as_float(p[0]) + __uint_as_float(p[1]);
+  }
+  {
+    const auto p = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = __uint_as_float(p[0]) + __uint_as_float(p[1]);
+  }
+  v = v + __uint_as_float(row_ror32<8>(__float_as_uint(v)));
+  v = v + __uint_as_float(row_ror32<4>(__float_as_uint(v)));
+  v = v + __uint_as_float(row_ror32<2>(__float_as_uint(v)));
+  v = v + __uint_as_float(row_ror32<1>(__float_as_uint(v)));
+  return v;
 }
 // wave maximum of a float (uniform result): DPP rotations within rows of 16, then the four row maxima
 __device__ __forceinline__ float wave_max_dpp(float v) {
@@ -234,98 +207,72 @@ __device__ __forceinline__ float wave_max_dpp(float v) {
   const float r3 = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__float_as_uint(v), 48));
   return fmaxf(fmaxf(r0, r1), fmaxf(r2, r3));
 }
-// wave maximum of a 64-bit value (uniform result), the same way
-__device__ __forceinline__ uint64_t wave_max_u64_dpp(uint64_t v) {
-  auto step = [&](uint64_t o) { v = o > v ? o : v; };
-  step(((uint64_t)row_ror32<1>((uint32_t)(v >> 32)) << 32) | row_ror32<1>((uint32_t)v));
-  step(((uint64_t)row_ror32<2>((uint32_t)(v >> 32)) << 32) | row_ror32<2>((uint32_t)v));
-  step(((uint64_t)row_ror32<4>((uint32_t)(v >> 32)) << 32) | row_ror32<4>((uint32_t)v));
-  step(((uint64_t)row_ror32<8>((uint32_t)(v >> 32)) << 32) | row_ror32<8>((uint32_t)v));
-  uint64_t best = 0;
-#pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    const uint64_t x = ((uint64_t)(uint32_t)__builtin_amdgcn_readlane((uint32_t)(v >> 32), 16 * r) << 32) |
-                       (uint32_t)__builtin_amdgcn_readlane((uint32_t)v, 16 * r);
-    best = x > best ? x : best;
-  }
-  return best;
+// wave maximum of an int, the same way
+__device__ __forceinline__ int wave_max_i32(int v) {
+  v = std::max(v, (int)row_ror32<1>((uint32_t)v));
+  v = std::max(v, (int)row_ror32<2>((uint32_t)v));
+  v = std::max(v, (int)row_ror32<4>((uint32_t)v));
+  v = std::max(v, (int)row_ror32<8>((uint32_t)v));
+  const int r0 = __builtin_amdgcn_readlane(v, 0), r1 = __builtin_amdgcn_readlane(v, 16);
+  const int r2 = __builtin_amdgcn_readlane(v, 32), r3 = __builtin_amdgcn_readlane(v, 48);
+  return std::max(std::max(r0, r1), std::max(r2, r3));
+}
+// sum of an int over the wave (uniform result)
+__device__ __forceinline__ int wave_sum_i32(int v) {
+  v += (int)row_ror32<1>((uint32_t)v);
+  v += (int)row_ror32<2>((uint32_t)v);
+  v += (int)row_ror32<4>((uint32_t)v);
+  v += (int)row_ror32<8>((uint32_t)v);
+  return __builtin_amdgcn_readlane(v, 0) + __builtin_amdgcn_readlane(v, 16) + __builtin_amdgcn_readlane(v, 32) +
+         __builtin_amdgcn_readlane(v, 48);
+}
+// inclusive prefix sum over the lanes: within rows of 16, then the row totals handed on
+template <int CTRL, int ROWS>
+__device__ __forceinline__ int dpp_add(int v) {
+  return v + __builtin_amdgcn_update_dpp(0, v, CTRL, ROWS, 0xF, false);
+}
+__device__ __forceinline__ int wave_scan_i32(int v) {
+  v = dpp_add<0x111, 0xF>(v);  // row_shr:1, 2, 4, 8
+  v = dpp_add<0x112, 0xF>(v);
+  v = dpp_add<0x114, 0xF>(v);
+  v = dpp_add<0x118, 0xF>(v);
+  v = dpp_add<0x142, 0xA>(v);  // row_bcast:15 into rows 1 and 3
+  v = dpp_add<0x143, 0xC>(v);  // row_bcast:31 into rows 2 and 3
+  return v;
 }
 
-// The k-th largest of the 64 lane values v < 2^BITS (0 = no value): the largest t with #{lanes: v >= t} >= k,
-// found bit by bit from the top with ballots; 0 when fewer than k lanes hold a value. Wave-uniform.
-template <int BITS = 32>
-__device__ __forceinline__ uint32_t wave_kth_largest(uint32_t v, int k) {
-  uint32_t t = 0;
-#pragma unroll
-  for (int bit = BITS - 1; bit >= 0; --bit) {
-    const uint32_t c = t | (1u << bit);
-    if (__builtin_popcountll(__builtin_amdgcn_ballot_w64(v >= c)) >= k) t = c;
-  }
-  return t;
+// ---- keys -----------------------------------------------------------------------------------------------
+// Selection keys are the bf16 bit patterns as signed 16-bit numbers with the magnitude bits of negative values
+// flipped (larger value = larger key; -0 has key -1, right below +0). For patterns without the sign bit the key is
+// the pattern itself.
+constexpr int KEY_MIN = -32768;
+__device__ __forceinline__ uint32_t keys2(uint32_t pair) {  // two at once
+  const i16x2 s = __builtin_bit_cast(i16x2, pair) >> (i16x2){15, 15};
+  return pair ^ (__builtin_bit_cast(uint32_t, s) & 0x7FFF7FFFu);
 }
-// the same for 32-bit values in two 16-bit halves: the low halves only decide among the lanes tied at the
-// boundary, and only when more of them are tied than are still needed
-__device__ __forceinline__ uint32_t wave_kth_largest32s(uint32_t v, int k) {
-  const uint32_t hi = v >> 16;
-  const uint32_t th = wave_kth_largest<16>(hi, k);
-  const int above = __builtin_popcountll(__builtin_amdgcn_ballot_w64(hi > th));
-  const int tied = __builtin_popcountll(__builtin_amdgcn_ballot_w64(hi == th));
-  const int need = k - above;
-  uint32_t tl = 0;
-  if (tied > need) tl = wave_kth_largest<16>(hi == th ? (v & 0xFFFFu) : 0u, need);
-  return (th << 16) | tl;
+__device__ __forceinline__ int key1(uint16_t b) { return (int)(int16_t)(b ^ (((int16_t)b >> 15) & 0x7FFF)); }
+__device__ __forceinline__ uint32_t max2(uint32_t a, uint32_t b) {
+  return __builtin_bit_cast(uint32_t,
+                            __builtin_elementwise_max(__builtin_bit_cast(i16x2, a), __builtin_bit_cast(i16x2, b)));
 }
-// the same for 64-bit values in two 32-bit halves
-__device__ __forceinline__ uint64_t wave_kth_largest64(uint64_t v, int k) {
-  const uint32_t hi = (uint32_t)(v >> 32);
-  const uint32_t th = wave_kth_largest(hi, k);
-  const int above = __builtin_popcountll(__builtin_amdgcn_ballot_w64(hi > th));
-  const int tied = __builtin_popcountll(__builtin_amdgcn_ballot_w64(hi == th));
-  const int need = k - above;
-  uint32_t tl = 0;
-  if (tied > need) tl = wave_kth_largest(hi == th ? (uint32_t)v : 0u, need);
-  return ((uint64_t)th << 32) | tl;
+// candidate key: larger = better (value descending, then token id ascending); never 0
+__device__ __forceinline__ uint64_t cand_key(uint16_t raw, uint32_t idx) {
+  return ((uint64_t)float_order_key(bf2f(raw) + 0.0f) << 32) | (uint64_t)(0xFFFFFFFFu - idx);
+}
+__device__ __forceinline__ float key_value(uint64_t key) {
+  const uint32_t hi = (uint32_t)(key >> 32);
+  return __uint_as_float((hi & 0x80000000u) ? (hi & 0x7FFFFFFFu) : ~hi);
 }
 
-// Piece keys are 32-bit: the upper half is the order key of the bf16 value (the upper 16 bits of
-// float_order_key of the widened value; its lower 16 bits are 0 for positive and 0xFFFF for negative values,
-// so nothing is lost), the lower half is 0xFFFF minus the element's index within the piece. Larger key =
-// larger value, then smaller token id; keys are unique within a piece and never 0 (0 marks an empty lane).
-__device__ __forceinline__ uint32_t piece_key(uint16_t raw, int local_idx) {
-  const uint32_t b = __float_as_uint(bf2f(raw) + 0.0f);
-  const uint32_t flip = (uint32_t)((int32_t)b >> 31) | 0x80000000u;
-  return ((b ^ flip) & 0xFFFF0000u) | (uint32_t)(0xFFFF - local_idx);
-}
-// the 64-bit candidate key (cand_key) of a piece key, the piece starting at row element c0
-__device__ __forceinline__ uint64_t global_key(uint32_t ck, int64_t c0) {
-  const uint32_t hi = (ck & 0xFFFF0000u) | ((ck & 0x80000000u) ? 0u : 0xFFFFu);
-  const int64_t idx = c0 + (0xFFFF - (int)(ck & 0xFFFFu));
-  return ((uint64_t)hi << 32) | (uint64_t)(0xFFFFFFFFu - (uint32_t)idx);
-}
-// 16-bit order key of a widened bf16 value (larger value -> larger key; -0 counts as +0)
-__device__ __forceinline__ uint32_t key16(float x) { return float_order_key(x + 0.0f) >> 16; }
-// the smallest widened bf16 value whose key16 is t
-__device__ __forceinline__ float key16_value(uint32_t t) {
-  return __uint_as_float(((t & 0x8000u) ? (t & 0x7FFFu) : (~t & 0xFFFFu)) << 16);
-}
-// Number of the n keys in buf (LDS, 16-byte aligned, zero-padded to a multiple of 4) larger than v; every lane
-// reads the same addresses (LDS broadcast).
-__device__ __forceinline__ int count_greater(uint32_t v, const uint32_t* buf, int n) {
-  int c = 0;
-  for (int j = 0; j < n; j += 4) {
-    const u32x4 x = *reinterpret_cast<const u32x4*>(buf + j);
-    c += (x[0] > v ? 1 : 0) + (x[1] > v ? 1 : 0) + (x[2] > v ? 1 : 0) + (x[3] > v ? 1 : 0);
-  }
-  return c;
-}
-
-struct FinalArgs {
-  int rows, k;
+struct TopkArgs {
+  const uint16_t* logits;
+  int64_t row_stride;
+  int rows, V, k;
   int npieces;         // (m, S) pairs per row
-  int nlists;          // candidate lists of k keys per row
-  const float* ws_m;
-  const double* ws_s;
-  const uint64_t* ws_cand;
+  int ng;              // group keys per piece: 16 (128 elements each), 4 (512 each) for k < 4
+  float* ws_m;         // [rows * npieces]
+  double* ws_s;        // [rows * npieces]
+  int16_t* ws_g;       // [rows * npieces * ng] the largest key1 of each group, in index order
   float* out_logp;     // [rows, k]
   void* out_ids;       // [rows, k] int32 or int64
   int ids_int64;
@@ -333,281 +280,12 @@ struct FinalArgs {
   const int32_t* vocab_ids;  // [V] token id of each logit column, or null (column = token id)
 };
 
-struct ChunkArgs {
-  const uint16_t* logits;
-  int64_t row_stride;
-  int rows, V, k;
-  int npieces;        // pieces of PIECE elements per row
-  int nchunks;        // chunks of CHUNK elements per row (the k > 32 kernel)
-  float* ws_m;        // [rows * npieces]
-  double* ws_s;       // [rows * npieces]
-  uint64_t* ws_cand;  // [rows * npieces * k] (k <= 32) or [rows * nchunks * k] (k > 32)
-};
-
-// ---- kernel 1, k > 32 -----------------------------------------------------------------------------------
-// One workgroup per (row, chunk of 8192 elements); wave w holds piece 4 chunk + w (its elements
-// 512 j + 8 lane + e of the piece, raw[j][e]) and writes that piece's maximum and sum.
-template <int KT>
-__global__ __launch_bounds__(NT) void topk_logz_chunk_kernel(ChunkArgs a) {
-  __shared__ uint64_t wcand[NT / 64][KMAX];
-  __shared__ __attribute__((aligned(16))) float etab[ETAB];
-  static_assert(NT == 256, "four pieces per chunk");
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
-  const int w = tid >> 6;
-  const int row = blockIdx.x / a.nchunks;
-  const int chunk = blockIdx.x % a.nchunks;
-  const int piece = 4 * chunk + w;
-  const int64_t p0 = (int64_t)piece * PIECE;
-  const uint16_t* src = a.logits + (int64_t)row * a.row_stride;
-  etab_stage(etab, NT / 64);
-
-  // element (j, e) of this thread: index p0 + 512 j + 8 lane + e (increasing with (j, e))
-  u16x8 raw[PER / 8];
-#pragma unroll
-  for (int j = 0; j < PER / 8; ++j) {
-    const int64_t i0 = p0 + 512 * j + 8 * lane;
-    if (i0 + 8 <= a.V) {
-      raw[j] = *reinterpret_cast<const u16x8*>(src + i0);
-    } else {
-#pragma unroll
-      for (int e = 0; e < 8; ++e) raw[j][e] = (i0 + e < a.V) ? src[i0 + e] : (uint16_t)0xFF80u;  // -inf
-    }
-  }
-  float mx = -INFINITY;
-  uint64_t list[KT];
-#pragma unroll
-  for (int i = 0; i < KT; ++i) list[i] = 0;
-#pragma unroll
-  for (int j = 0; j < PER / 8; ++j)
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const float x = bf2f(raw[j][e]);
-      mx = fmaxf(mx, x);
-      const int64_t idx = p0 + 512 * j + 8 * lane + e;
-      if (idx < a.V) {
-        uint64_t key = cand_key(x, (uint32_t)idx);
-        if (key > list[KT - 1]) {
-          // insertion into the descending list (unrolled compare-and-shift)
-#pragma unroll
-          for (int s = 0; s < KT; ++s) {
-            const uint64_t cur = list[s];
-            const bool take = key > cur;
-            list[s] = take ? key : cur;
-            key = take ? cur : key;
-          }
-        }
-      }
-    }
-  const float m = wave_max_dpp(mx);
-  __builtin_amdgcn_s_waitcnt(0);  // this wave's part of the table has landed
-  __syncthreads();
-  const int nvalid = (int)std::max<int64_t>(0, std::min<int64_t>((int64_t)PIECE, (int64_t)a.V - p0));
-  const float ssum = wave_sum_tree(piece_lane_sum(raw, m, src + p0, nvalid, etab));
-  if (lane == 0 && piece < a.npieces) {
-    const int64_t ps = (int64_t)row * a.npieces + piece;
-    a.ws_m[ps] = m;
-    a.ws_s[ps] = (double)ssum;
-  }
-  // per-wave top-k, then the first wave merges the 4 wave lists
-  wave_topk<KT>(list, a.k, wcand[w]);
-  __syncthreads();
-  const int64_t slot = (int64_t)row * a.nchunks + chunk;
-  if (w == 0) {
-    // the 4 waves' k candidates, spread over the lanes as sorted per-lane lists (at most 4 k / 64 <= 16 per
-    // lane), then k rounds of argmax
-    uint64_t l2[KT];
-#pragma unroll
-    for (int i = 0; i < KT; ++i) l2[i] = 0;
-    for (int t = lane; t < (NT / 64) * a.k; t += 64) {
-      uint64_t key = wcand[t % (NT / 64)][t / (NT / 64)];
-#pragma unroll
-      for (int s = 0; s < KT; ++s) {
-        const uint64_t cur = l2[s];
-        const bool take = key > cur;
-        l2[s] = take ? key : cur;
-        key = take ? cur : key;
-      }
-    }
-    uint64_t* out = a.ws_cand + slot * a.k;
-    int head = 0;
-    for (int i = 0; i < a.k; ++i) {
-      uint64_t mine = 0;
-#pragma unroll
-      for (int j = 0; j < KT; ++j)
-        if (j == head) mine = l2[j];
-      const uint64_t best = wave_max_u64(mine);
-      if (best != 0 && mine == best) ++head;
-      if (lane == 0) out[i] = best;
-    }
-  }
-}
-
-// ---- kernel 1, k <= 32 ----------------------------------------------------------------------------------
-// One wave per piece, PW waves per workgroup sharing the table; a wave takes pieces (blockIdx.x * PW + wave) +
-// i * gridDim.x * PW (piece id = row * npieces + piece). t_w, the k-th largest 16-bit value key of the 64 lane
-// maxima, is reached by the piece's top k (k lanes reach it); the 8-element groups whose maximum reaches t_w
-// are listed in LDS; the 32-bit keys of their elements with value keys >= t_w are formed one per lane (at most
-// 8 listed groups; otherwise a running top k in 64-lane passes) and ranked by counting. Without ties at t_w
-// fewer than 4 (k - 1) + 4 groups are listed, typically about k; with many ties up to all 256 (slower, still
-// exact).
-constexpr int PW = 16;  // waves per workgroup
-// the row merge of kernel 2 for k <= 8 and at most 128 lists, by one wave (defined with kernel 2)
-__device__ void final_row_fast(const FinalArgs& a, int row, double* terms);
-// ROW: one workgroup per row of at most PW pieces (wave w takes piece w), and the workgroup's wave 0 merges
-// the row once its pieces are written (no second kernel); otherwise kernel 2 merges
-template <int KS, bool ROW>
-__global__ __launch_bounds__(PW * 64) __attribute__((amdgpu_waves_per_eu(ROW ? 4 : 8))) void topk_piece_kernel(
-    ChunkArgs a, FinalArgs f) {
-  constexpr int CAPR = 8;  // listed groups whose raw values are staged in LDS (one 64-lane pass)
-  __shared__ __attribute__((aligned(16))) float etab[ETAB];
-  __shared__ uint16_t gfirst[PW][256];   // piece index of each listed group's first element
-  __shared__ u16x8 graw[PW][CAPR];       // raw values of the first CAPR listed groups
-  __shared__ __attribute__((aligned(16))) uint32_t keep_buf[PW][64];
-  const int lane = threadIdx.x & 63;
-  // the wave index in a scalar register: as a vector value it makes the per-wave LDS bases vector values too,
-  // and at the 64-VGPR budget of eight waves per SIMD four of them spilled (scratch reloads on every piece)
-  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int k = a.k;
-  const int total = a.rows * a.npieces;
-  etab_stage(etab, PW);
-  bool staged = false;  // every wave passes the one barrier that publishes the table exactly once
-  const int pid0 = ROW ? (w < a.npieces ? (int)blockIdx.x * a.npieces + w : total) : (int)blockIdx.x * PW + w;
-  const int pstep = ROW ? total : (int)gridDim.x * PW;
-  for (int pid = pid0; pid < total; pid += pstep) {
-    const int row = pid / a.npieces;
-    const int64_t p0 = (int64_t)(pid - row * a.npieces) * PIECE;
-    const uint16_t* psrc = a.logits + (int64_t)row * a.row_stride + p0;
-    const int nvalid = (int)std::min<int64_t>((int64_t)PIECE, (int64_t)a.V - p0);
-    // group j: piece elements 512 j + 8 lane + e; past the row end they read as -inf
-    u16x8 raw[4];
-    if (nvalid == PIECE) {
-#pragma unroll
-      for (int j = 0; j < 4; ++j) raw[j] = *reinterpret_cast<const u16x8*>(psrc + 512 * j + 8 * lane);
-    } else {
-      // the row's last piece: a group starting before the row end is read whole (the buffer holds
-      // rows * row_stride elements, row_stride a multiple of 8), its elements past the end set to -inf
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int i0 = 512 * j + 8 * lane;
-        u16x8 x = {0xFF80u, 0xFF80u, 0xFF80u, 0xFF80u, 0xFF80u, 0xFF80u, 0xFF80u, 0xFF80u};
-        if (i0 < nvalid) x = *reinterpret_cast<const u16x8*>(psrc + i0);
-#pragma unroll
-        for (int e = 0; e < 8; ++e) x[e] = (i0 + e < nvalid) ? x[e] : (uint16_t)0xFF80u;
-        raw[j] = x;
-      }
-    }
-    // group maxima (widened floats), the lane maximum, the piece maximum and the threshold
-    float gm[4];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const u32x4 u = __builtin_bit_cast(u32x4, raw[j]);
-      float x = -INFINITY;
-#pragma unroll
-      for (int q = 0; q < 4; ++q) x = fmaxf(x, fmaxf(__uint_as_float(u[q] << 16), __uint_as_float(u[q] & 0xFFFF0000u)));
-      gm[j] = x;
-    }
-    const float lmax = fmaxf(fmaxf(gm[0], gm[1]), fmaxf(gm[2], gm[3]));
-    const uint32_t tw = wave_kth_largest<16>(key16(lmax), k);
-    const float m = wave_max_dpp(lmax);
-    const float tv = key16_value(tw);
-    // list the groups that may hold candidates (ballot + lane rank)
-    int ng = 0;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const bool take = gm[j] >= tv;
-      const uint64_t mk = __builtin_amdgcn_ballot_w64(take);
-      if (mk) {
-        if (take) {
-          const int pos = ng + (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(mk >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mk, 0));
-          gfirst[w][pos] = (uint16_t)(512 * j + 8 * lane);
-          if (pos < CAPR) graw[w][pos] = raw[j];
-        }
-        ng += __builtin_popcountll(mk);
-      }
-    }
-    if (!staged) {
-      __builtin_amdgcn_s_waitcnt(0);  // this wave's part of the table has landed
-      __syncthreads();
-      staged = true;
-    }
-    // S_c before the selection, so that the raw values are dead during it
-    const float ssum = wave_sum_tree(piece_lane_sum(raw, m, psrc, nvalid, etab));
-    __builtin_amdgcn_wave_barrier();
-    // element i of the listed groups is group i / 8, element i % 8
-    auto fetch = [&](int i) -> uint32_t {
-      if (i >= 8 * ng) return 0u;
-      const int g = i >> 3;
-      const int idx = (int)gfirst[w][g] + (i & 7);
-      if (idx >= nvalid) return 0u;
-      const uint16_t r = g < CAPR ? graw[w][g][i & 7] : psrc[idx];
-      const uint32_t key = piece_key(r, idx);
-      return (key >> 16) >= tw ? key : 0u;
-    };
-    uint32_t v = fetch(lane);
-    uint64_t live;
-    if (ng <= CAPR) {
-      live = __builtin_amdgcn_ballot_w64(v != 0u);
-    } else {
-      // running top k: lanes hold the kept keys (low lanes) and the next unseen candidates
-      int next = 64;
-      for (;;) {
-        const uint32_t t = wave_kth_largest32s(v, k);
-        live = __builtin_amdgcn_ballot_w64(v != 0u && v >= t);
-        if (next >= 8 * ng) break;
-        const int nk = __builtin_popcountll(live);
-        if ((live >> lane) & 1ull)
-          keep_buf[w][__builtin_amdgcn_mbcnt_hi((uint32_t)(live >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)live, 0))] = v;
-        __builtin_amdgcn_wave_barrier();
-        v = lane < nk ? keep_buf[w][lane] : fetch(next + lane - nk);
-        __builtin_amdgcn_wave_barrier();
-        next += 64 - nk;
-      }
-    }
-    // rank of each kept key among the kept keys (compacted into LDS, zero-padded to a multiple of 4); the
-    // piece's list is written in rank order, zeros after its last key
-    const bool kept = (live >> lane) & 1ull;
-    const int nl = __builtin_popcountll(live);
-    __builtin_amdgcn_wave_barrier();
-    if (kept) keep_buf[w][__builtin_amdgcn_mbcnt_hi((uint32_t)(live >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)live, 0))] = v;
-    if (lane >= nl && lane < ((nl + 3) & ~3)) keep_buf[w][lane] = 0u;
-    __builtin_amdgcn_wave_barrier();
-    const int rank = kept ? count_greater(v, keep_buf[w], nl) : 64;
-    uint64_t* out = a.ws_cand + (int64_t)pid * k;
-    if (rank < k) out[rank] = global_key(v, p0);
-    if (lane >= nl && lane < k) out[lane] = 0;
-    if (lane == 0) {
-      a.ws_m[pid] = m;
-      a.ws_s[pid] = (double)ssum;
-    }
-  }
-  if (!staged) {
-    __builtin_amdgcn_s_waitcnt(0);
-    __syncthreads();
-  }
-  if constexpr (ROW) {
-    __shared__ double fterms[PW];
-    __syncthreads();  // the row's piece lists, maxima and sums are written (the barrier orders global memory
-                      // within the workgroup)
-    if (w == 0) final_row_fast(f, blockIdx.x, fterms);
-  }
-}
-
-// ---- kernel 2 -------------------------------------------------------------------------------------------
-
-constexpr int FINAL_CAND = 8192;  // candidates of one row staged in LDS by the k > 32 merge (nlists * k)
-
-__device__ __forceinline__ float key_value(uint64_t key) {
-  const uint32_t hi = (uint32_t)(key >> 32);
-  return __uint_as_float((hi & 0x80000000u) ? (hi & 0x7FFFFFFFu) : ~hi);
-}
-
 // The (m, S) of the row's first 256 pieces, piece c in lane c % 64, entry c / 64 (loaded before they are needed).
 struct PieceSums {
   float m[4];
   double s[4];
 };
-__device__ __forceinline__ PieceSums load_piece_sums(const FinalArgs& a, int row) {
+__device__ __forceinline__ PieceSums load_piece_sums(const TopkArgs& a, int row) {
   const int lane = threadIdx.x & 63;
   const int np = a.npieces;
   PieceSums p;
@@ -622,7 +300,7 @@ __device__ __forceinline__ PieceSums load_piece_sums(const FinalArgs& a, int row
 // log Z of row `row` from its pieces' (m, S), formed by one wave: the terms S_c exp_det(m_c - m) in parallel,
 // added in piece order by a chain of lane reads (pieces past 256 through LDS scratch `terms` of npieces
 // doubles); wave-uniform result.
-__device__ float row_logz(const FinalArgs& a, int row, const PieceSums& p, double* terms) {
+__device__ float row_logz(const TopkArgs& a, int row, const PieceSums& p, double* terms) {
 #pragma clang fp contract(off)
   const int lane = threadIdx.x & 63;
   const int np = a.npieces;
@@ -669,204 +347,503 @@ __device__ float row_logz(const FinalArgs& a, int row, const PieceSums& p, doubl
   return (float)((double)m + log_det(z));
 }
 
+// ---- the top k of a row's candidates ----------------------------------------------------------------------
+constexpr int NBIN = 1024;
+constexpr int COUNT_MAX = 256;  // up to here a candidate's rank is counted against all others
+constexpr int CAND_MAX = 1024;
+struct MergeLds {
+  uint32_t hist[NBIN];
+  __attribute__((aligned(16))) uint64_t cand[CAND_MAX + 2];
+  __attribute__((aligned(16))) uint64_t sel[KMAX];
+  uint16_t bnd[CAND_MAX];
+  uint16_t glist[2 * KMAX];  // the groups whose elements are looked at
+  int wsum[16];
+  int count[40];
+  int n, nsel, nb, bin, need, ng, top;
+  float logz;
+};
 
-// k <= 8, at most 128 lists: each lane's (up to two) lists in registers; k rounds of "the largest head wins, its
-// list shifts up by one entry"; winner i is kept by lane i, and the k outputs are written together once log Z
-// is known. One wave; `terms`: LDS scratch of npieces doubles.
-__device__ void final_row_fast(const FinalArgs& a, int row, double* terms) {
+__device__ __forceinline__ void put_one(const TopkArgs& a, int row, int pos, uint64_t key, float logz) {
+  uint32_t idx = 0xFFFFFFFFu - (uint32_t)key;
+  if (a.vocab_ids) idx = (uint32_t)a.vocab_ids[idx];
+  a.out_logp[(int64_t)row * a.k + pos] = key_value(key) - logz;
+  if (a.ids_int64)
+    static_cast<int64_t*>(a.out_ids)[(int64_t)row * a.k + pos] = (int64_t)idx;
+  else
+    static_cast<int32_t*>(a.out_ids)[(int64_t)row * a.k + pos] = (int32_t)idx;
+}
+
+// The bin b that holds the k-th largest of the histogrammed values and how many of that bin are needed, by one wave:
+// lane l holds bins 16 (63 - l) .. + 15, an inclusive scan over the lanes gives the suffix sums. False (every lane) if
+// fewer than k values are histogrammed.
+__device__ __forceinline__ bool kth_bin(const uint32_t* hist, int k, int* bin, int* need) {
   const int lane = threadIdx.x & 63;
-  const int k = a.k;
-  const int nls = a.nlists;
-  const uint64_t* src = a.ws_cand + (int64_t)row * nls * k;
-  const PieceSums ps = load_piece_sums(a, row);
-  auto put = [&](int pos, uint64_t key, float logz) {
-    const float x = key ? key_value(key) : -INFINITY;
-    uint32_t idx = key ? 0xFFFFFFFFu - (uint32_t)key : 0u;
-    if (key && a.vocab_ids) idx = (uint32_t)a.vocab_ids[idx];
-    a.out_logp[(int64_t)row * k + pos] = x - logz;
-    if (a.ids_int64)
-      static_cast<int64_t*>(a.out_ids)[(int64_t)row * k + pos] = (int64_t)idx;
-    else
-      static_cast<int32_t*>(a.out_ids)[(int64_t)row * k + pos] = (int32_t)idx;
-  };
-  uint64_t l0[8], l1[8];
+  const int b0 = 16 * (63 - lane);
+  int h[16];
 #pragma unroll
-  for (int j = 0; j < 8; ++j) {
-    l0[j] = (lane < nls && j < k) ? src[lane * k + j] : 0ull;
-    l1[j] = (lane + 64 < nls && j < k) ? src[(lane + 64) * k + j] : 0ull;
+  for (int i = 0; i < 16; i += 4) {
+    const u32x4 x = *reinterpret_cast<const u32x4*>(hist + b0 + i);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) h[i + e] = (int)x[e];
   }
-  uint64_t win = 0ull;
-  for (int i = 0; i < k; ++i) {
-    const uint64_t mine = l0[0] > l1[0] ? l0[0] : l1[0];
-    const uint64_t best = wave_max_u64_dpp(mine);
-    if (lane == i) win = best;
-    if (best != 0ull && mine == best) {  // keys are unique (they contain the token id)
-      if (l0[0] == best) {
+  int own = 0;
 #pragma unroll
-        for (int j = 0; j < 7; ++j) l0[j] = l0[j + 1];
-        l0[7] = 0ull;
-      } else {
+  for (int i = 0; i < 16; ++i) own += h[i];
+  const int inc = wave_scan_i32(own);
+  const bool here = inc >= k && inc - own < k;  // one lane, if any
+  if (here) {
+    int above = inc - own, b = -1;
 #pragma unroll
-        for (int j = 0; j < 7; ++j) l1[j] = l1[j + 1];
-        l1[7] = 0ull;
+    for (int i = 15; i >= 0; --i) {
+      if (b < 0) {
+        if (above + h[i] >= k)
+          b = b0 + i;
+        else
+          above += h[i];
       }
     }
+    *bin = b;
+    *need = k - above;
   }
-  const float logz = row_logz(a, row, ps, terms);
-  if (lane < k) put(lane, win, logz);
-  if (lane == 0 && a.out_logz) a.out_logz[row] = logz;
+  return __builtin_amdgcn_ballot_w64(here) != 0;
 }
 
-// k > 32: one wave per row, k rounds of wave argmax over the row's candidates
-__global__ __launch_bounds__(64) void topk_logz_final_kernel(FinalArgs a) {
-  __shared__ uint64_t cand[FINAL_CAND];
-  __shared__ double terms[FINAL_CAND / 4];
-  const int row = blockIdx.x;
-  const int lane = threadIdx.x;
-  const int n = a.nlists * a.k;
-  const uint64_t* src = a.ws_cand + (int64_t)row * n;
-  const PieceSums ps = load_piece_sums(a, row);
-  for (int t = lane; t < n; t += 64) cand[t] = src[t];
-  const float logz = row_logz(a, row, ps, terms);
-  // keys are unique (they contain the token id), the winner is removed
-  for (int i = 0; i < a.k; ++i) {
-    uint64_t mine = 0;
-    int where = -1;
-    for (int t = lane; t < n; t += 64) {
-      const uint64_t c = cand[t];
-      if (c > mine) {
-        mine = c;
-        where = t;
-      }
-    }
-    const uint64_t best = wave_max_u64(mine);
-    if (best != 0 && mine == best) cand[where] = 0;
-    if (lane == 0) {
-      const float x = best ? key_value(best) : -INFINITY;
-      uint32_t idx = best ? 0xFFFFFFFFu - (uint32_t)best : 0u;
-      if (best && a.vocab_ids) idx = (uint32_t)a.vocab_ids[idx];
-      a.out_logp[(int64_t)row * a.k + i] = x - logz;
-      if (a.ids_int64)
-        static_cast<int64_t*>(a.out_ids)[(int64_t)row * a.k + i] = (int64_t)idx;
-      else
-        static_cast<int32_t*>(a.out_ids)[(int64_t)row * a.k + i] = (int32_t)idx;
-    }
-  }
-  if (lane == 0 && a.out_logz) a.out_logz[row] = logz;
-}
-
-// k <= 32: one wave per row. The row's top k are merged from the pieces' rank-ordered lists (up to 128 lists:
-// two list heads per lane, k rounds of "the largest head is output and its list advances"), or, for more
-// lists, kept over all candidates in 64-lane passes (64-bit keys) and then ranked.
-__global__ __launch_bounds__(64) void topk_small_final_kernel(FinalArgs a) {
-  extern __shared__ __align__(16) unsigned char fsm[];
-  double* terms = reinterpret_cast<double*>(fsm);  // [npieces]
-  uint64_t* keep_buf = reinterpret_cast<uint64_t*>(terms + a.npieces);  // [64]
-  uint64_t* cand = keep_buf + 64;  // [nlists k] when nlists k <= FINAL_STAGE: the row's candidates
-  const int row = blockIdx.x;
-  const int lane = threadIdx.x;
+// Called by all NTH threads of a workgroup, after a barrier, with n >= k candidates in ml.cand and log Z in ml.logz;
+// top: the largest candidate's 16-bit value key. Few candidates (what k <= 32 nearly always leaves) are ranked by
+// counting, n broadcast reads each. More: the value keys' distance from the largest, clamped to 1024 bins, is
+// histogrammed, the bin that holds the k-th largest is read off the suffix sums, the candidates above it are taken,
+// those in it by their rank among themselves (one value unless clamped, so ties by token id), and the k taken are
+// ranked by counting, four threads each.
+template <int NTH>
+__device__ void merge_row(const TopkArgs& a, int row, int n, int top, MergeLds& ml) {
+  const int tid = threadIdx.x;
   const int k = a.k;
-  const int nls = a.nlists;
-  const int n = nls * k;
-  const uint64_t* src = a.ws_cand + (int64_t)row * n;
-  auto put = [&](int pos, uint64_t key, float logz) {
-    const float x = key ? key_value(key) : -INFINITY;
-    uint32_t idx = key ? 0xFFFFFFFFu - (uint32_t)key : 0u;
-    if (key && a.vocab_ids) idx = (uint32_t)a.vocab_ids[idx];
-    a.out_logp[(int64_t)row * k + pos] = x - logz;
-    if (a.ids_int64)
-      static_cast<int64_t*>(a.out_ids)[(int64_t)row * k + pos] = (int64_t)idx;
-    else
-      static_cast<int32_t*>(a.out_ids)[(int64_t)row * k + pos] = (int32_t)idx;
-  };
-  const PieceSums ps = load_piece_sums(a, row);
-  if (nls <= 128 && k <= 8) {
-    final_row_fast(a, row, terms);
+  uint64_t* cand = ml.cand;
+  const float logz = ml.logz;
+  if (tid == 0 && a.out_logz) a.out_logz[row] = logz;
+  if (n <= COUNT_MAX) {
+    if (tid < n) {
+      const uint64_t v = cand[tid];
+      int r = 0;
+      for (int i = 0; i < n; i += 2) {
+        const u64x2 x = *reinterpret_cast<const u64x2*>(cand + i);
+        r += (x[0] > v ? 1 : 0) + (x[1] > v && i + 1 < n ? 1 : 0);
+      }
+      if (r < k) put_one(a, row, r, v, logz);
+    }
     return;
   }
-  // the candidates are staged in LDS (four loads per lane in flight at a time, while log Z is formed), so
-  // that the merge below reads no global memory
-  const bool staged = n <= FINAL_STAGE;
-  if (staged) {
-    for (int i0 = 0; i0 < n; i0 += 256) {
-      uint64_t x[4];
-#pragma unroll
-      for (int r = 0; r < 4; ++r) x[r] = (i0 + 64 * r + lane < n) ? src[i0 + 64 * r + lane] : 0ull;
-#pragma unroll
-      for (int r = 0; r < 4; ++r)
-        if (i0 + 64 * r + lane < n) cand[i0 + 64 * r + lane] = x[r];
-    }
+  for (int i = tid; i < NBIN; i += NTH) ml.hist[i] = 0;
+  if (tid < KMAX) ml.sel[tid] = 0;
+  if (tid == 0) ml.nsel = ml.nb = 0;
+  auto bin_of = [&](uint64_t v) -> int {
+    const int d = NBIN - 1 - (top - (int)(v >> 48));
+    return d < 0 ? 0 : (d > NBIN - 1 ? NBIN - 1 : d);
+  };
+  __syncthreads();
+  for (int i = tid; i < n; i += NTH) atomicAdd(&ml.hist[bin_of(cand[i])], 1u);
+  __syncthreads();
+  if (tid < 64) kth_bin(ml.hist, k, &ml.bin, &ml.need);
+  __syncthreads();
+  const int bin = ml.bin, need = ml.need;
+  for (int i = tid; i < n; i += NTH) {
+    const uint64_t v = cand[i];
+    const int b = bin_of(v);
+    if (b > bin)
+      ml.sel[atomicAdd(&ml.nsel, 1)] = v;
+    else if (b == bin)
+      ml.bnd[atomicAdd(&ml.nb, 1)] = (uint16_t)i;
   }
-  const float logz = row_logz(a, row, ps, terms);
+  __syncthreads();
+  const int nb = ml.nb;
+  for (int i = tid; i < nb; i += NTH) {
+    const uint64_t v = cand[ml.bnd[i]];
+    int r = 0;
+    if (nb > need)
+      for (int j = 0; j < nb; ++j) r += cand[ml.bnd[j]] > v ? 1 : 0;
+    if (r < need) ml.sel[atomicAdd(&ml.nsel, 1)] = v;
+  }
+  __syncthreads();
+  // four threads per selected key: thread p of a key reads entries 8 i + 2 p, + 1
+  static_assert(NTH / 4 >= KMAX || NTH / 4 >= 32, "one pass");
+  const int s = tid >> 2;
+  const uint64_t v = s < k ? ml.sel[s] : 0ull;
+  int r = 0;
+  for (int i = 2 * (tid & 3); i < k; i += 8) {
+    const u64x2 x = *reinterpret_cast<const u64x2*>(ml.sel + i);
+    r += (x[0] > v ? 1 : 0) + (x[1] > v ? 1 : 0);
+  }
+  r += __builtin_amdgcn_update_dpp(0, r, 0xB1, 0xF, 0xF, false);  // lane ^ 1
+  r += __builtin_amdgcn_update_dpp(0, r, 0x4E, 0xF, 0xF, false);  // lane ^ 2
+  if (s < k && (tid & 3) == 0) put_one(a, row, r, v, logz);
+}
+
+// Kernel 2's work for one row, by all NTH threads of a workgroup, once the row's (m, S) and group keys are in memory.
+// The groups' keys are histogrammed by their distance from the largest (1024 bins, 8 octaves of bf16) and the k-th
+// largest, t, is read off the suffix sums (or found by bisection, where it lies further down). Listed are the groups
+// above t (fewer than k) and the first k of those at t in index order, which hold the first k elements equal to t:
+// nearly always k groups and a few, never more than 2 k. Their elements from t up are the candidates; should they not
+// fit (rows of ties, masked rows), the k-th largest key among the listed groups and the index of the last equal
+// element taken are found by bisection over counts. Wave 0 forms log Z while the others wait for the elements.
+// What bounds it: a chain of two trips to memory and about ten barriers. 128 rows, k = 8: 5.7 us (5.4 for merging
+// the pieces' top-8 lists); 120 rows, k = 256: 11.2 us (1.83 ms for 256 serial maxima over 7936 listed keys).
+template <int NTH>
+__device__ void row_topk(const TopkArgs& a, int row, MergeLds& ml, double* terms) {
+  constexpr int NW = NTH / 64;
+  constexpr int NQ = 4;  // loads of four keys held in registers per thread; further ones are read again in every pass
+  const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int k = a.k;
+  PieceSums ps;
+  if (w == 0) ps = load_piece_sums(a, row);
   if (k == 0) {
-    if (lane == 0 && a.out_logz) a.out_logz[row] = logz;
+    if (w == 0) {
+      const float z = row_logz(a, row, ps, terms);
+      if (lane == 0) a.out_logz[row] = z;
+    }
     return;
   }
-  __builtin_amdgcn_s_waitcnt(0);
-  __builtin_amdgcn_wave_barrier();
-  const uint64_t* cs = staged ? cand : src;
-  if (nls <= 128) {
-    int h0 = 0, h1 = 0;
-    const bool has0 = lane < nls, has1 = lane + 64 < nls;
-    uint64_t c0 = has0 ? cs[lane * k] : 0ull;
-    uint64_t c1 = has1 ? cs[(lane + 64) * k] : 0ull;
-    for (int i = 0; i < k; ++i) {
-      const uint64_t mine = c0 > c1 ? c0 : c1;
-      const uint64_t best = wave_max_u64_dpp(mine);
-      if (best != 0ull && mine == best) {  // keys are unique (they contain the token id)
-        if (c0 == best) {
-          ++h0;
-          c0 = h0 < k ? cs[lane * k + h0] : 0ull;
-        } else {
-          ++h1;
-          c1 = h1 < k ? cs[(lane + 64) * k + h1] : 0ull;
+  // thread t holds the groups [t gp, (t + 1) gp)
+  const int ngroups = a.npieces * a.ng;
+  const int gp = ((ngroups + NTH - 1) / NTH + 3) & ~3;
+  const uint64_t* gsrc = reinterpret_cast<const uint64_t*>(a.ws_g + (int64_t)row * ngroups);
+  const int g0 = tid * gp, g1 = std::min(ngroups, g0 + gp);
+  uint64_t kq[NQ];
+#pragma unroll
+  for (int c = 0; c < NQ; ++c) kq[c] = g0 + 4 * c < g1 ? gsrc[(g0 >> 2) + c] : 0ull;
+  auto for_groups = [&](auto visit) {  // visit(key, group)
+    auto four = [&](uint64_t q, int g) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) visit((int)(int16_t)(uint16_t)(q >> (16 * i)), g + i);
+    };
+#pragma unroll
+    for (int c = 0; c < NQ; ++c)
+      if (g0 + 4 * c < g1) four(kq[c], g0 + 4 * c);
+    for (int g = g0 + 4 * NQ; g < g1; g += 4) four(gsrc[g >> 2], g);
+  };
+  for (int i = tid; i < NBIN; i += NTH) ml.hist[i] = 0;
+  if (tid == 0) {
+    ml.n = 0;
+    ml.bin = -1;
+  }
+  if (tid < 40) ml.count[tid] = 0;
+  int top = KEY_MIN;
+  for_groups([&](int key, int) { top = std::max(top, key); });
+  top = wave_max_i32(top);
+  if (lane == 0) ml.wsum[w] = top;
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < NW; ++i) top = std::max(top, ml.wsum[i]);
+  for_groups([&](int key, int) {
+    const int d = NBIN - 1 - (top - key);
+    if (d >= 0) atomicAdd(&ml.hist[d], 1u);
+  });
+  __syncthreads();
+  if (w == 0) kth_bin(ml.hist, k, &ml.bin, &ml.need);
+  __syncthreads();
+  int t = top - (NBIN - 1 - ml.bin);
+  if (ml.bin < 0) {
+    // further down than the bins reach, or fewer than k groups (then the lowest key)
+    uint32_t T = 0;
+#pragma unroll 1
+    for (int bit = 15; bit >= 0; --bit) {
+      const int cut = (int)(T | (1u << bit)) - 32768;
+      int own = 0;
+      for_groups([&](int key, int) { own += key >= cut ? 1 : 0; });
+      own = wave_sum_i32(own);
+      if (lane == 0 && own) atomicAdd(&ml.count[bit], own);
+      __syncthreads();
+      if (ml.count[bit] >= k) T |= 1u << bit;
+    }
+    t = (int)T - 32768;
+    __syncthreads();
+    if (tid < 40) ml.count[tid] = 0;
+  }
+  if (t == 0) t = -1;  // -0 counts as 0
+  auto at_t = [&](int key) -> bool { return t == -1 ? key == 0 || key == -1 : key == t; };
+  // the list; both counts in one prefix sum (fewer than k groups above t, at most 2^15 at it)
+  int both = 0;
+  for_groups([&](int key, int) { both += at_t(key) ? 1 : key > t ? 1 << 16 : 0; });
+  const int inc = wave_scan_i32(both);
+  if (lane == 63) ml.wsum[w] = inc;
+  __syncthreads();
+  int before = inc - both, all = 0;
+#pragma unroll
+  for (int i = 0; i < NW; ++i) {
+    const int x = ml.wsum[i];
+    before += i < w ? x : 0;
+    all += x;
+  }
+  const int nabove = all >> 16, nl = nabove + std::min(all & 0xFFFF, k);
+  if (both) {
+    int pa = before >> 16, pe = before & 0xFFFF;
+    for_groups([&](int key, int g) {
+      if (at_t(key)) {
+        if (pe < k) ml.glist[nabove + pe] = (uint16_t)g;
+        ++pe;
+      } else if (key > t) {
+        ml.glist[pa++] = (uint16_t)g;
+      }
+    });
+  }
+  __syncthreads();
+  // The listed groups' elements, eight per lane and step: step u is 16 or 64 lanes' share of a group.
+  const uint16_t* src = a.logits + (int64_t)row * a.row_stride;
+  const int lsh = a.ng == 16 ? 4 : 6;
+  const int steps = nl << lsh;
+  auto start_of = [&](int u) -> int { return 8 * (((int)ml.glist[u >> lsh] << lsh) + (u & ((1 << lsh) - 1))); };
+  if (w == 0) {
+    const float z = row_logz(a, row, ps, terms);
+    if (lane == 0) ml.logz = z;
+  } else {
+    constexpr int ST = NTH - 64;
+    const i16x2 below = {(int16_t)(t - 1), (int16_t)(t - 1)};  // t > KEY_MIN here or every element is taken
+    for (int u0 = tid - 64 - lane; u0 < steps; u0 += 4 * ST) {
+      u32x4 x[4];
+      int i0[4];
+#pragma unroll
+      for (int h = 0; h < 4; ++h) {  // four loads in flight; past the list the row's first elements, not counted
+        const int u = u0 + lane + h * ST;
+        i0[h] = u < steps ? start_of(u) : a.V;
+        x[h] = *reinterpret_cast<const u32x4*>(src + (i0[h] < a.V ? i0[h] : 0));
+      }
+      uint32_t hits = 0;  // bit 8 h + e
+#pragma unroll
+      for (int h = 0; h < 4; ++h) {
+        uint32_t m = 0;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          // key > t - 1: the sign of the saturated difference, in both halves
+          const uint32_t d = __builtin_bit_cast(
+              uint32_t, __builtin_elementwise_sub_sat(below, __builtin_bit_cast(i16x2, keys2(x[h][q]))));
+          m |= (((d >> 15) & 1u) | ((d >> 30) & 2u)) << (2 * q);
+        }
+        if (t == KEY_MIN) m = 0xFFu;
+        const int rest = a.V - i0[h];
+        if (rest < 8) m &= rest <= 0 ? 0u : (1u << rest) - 1u;
+        hits |= m << (8 * h);
+      }
+      const int mine = __builtin_popcount(hits);
+      const int inc = wave_scan_i32(mine);
+      const int total = __builtin_amdgcn_readlane(inc, 63);
+      if (total == 0) continue;
+      int base = 0;
+      if (lane == 0) base = atomicAdd(&ml.n, total);
+      int pos = __builtin_amdgcn_readfirstlane(base) + inc - mine;
+      for (; hits && pos < CAND_MAX; hits &= hits - 1, ++pos) {
+        const int b = __builtin_ctz(hits);
+        const int idx = start_of(u0 + lane + (b >> 3) * ST) + (b & 7);
+        ml.cand[pos] = cand_key(src[idx], (uint32_t)idx);
+      }
+    }
+  }
+  __syncthreads();
+  int n = ml.n;
+  // (more than COUNT_MAX candidates for k <= 32 are ties, which the bisection settles sooner than counting them against
+  // each other: a row of 151936 equal values, k = 8, 37 against 86 us)
+  if (n > (k <= 32 ? COUNT_MAX : CAND_MAX)) {
+    auto norm = [](int key) -> int { return key == -1 ? 0 : key; };
+    auto elem = [](const u32x4& x, int e) -> uint16_t { return (uint16_t)((e & 1) ? x[e >> 1] >> 16 : x[e >> 1] & 0xFFFFu); };
+    auto for_elements = [&](auto visit) {  // visit(the eight elements, the index of the first)
+      for (int u = tid; u < steps; u += NTH) {
+        const int i0 = start_of(u);
+        if (i0 < a.V) visit(*reinterpret_cast<const u32x4*>(src + i0), i0);
+      }
+    };
+    auto count = [&](int slot, auto pred) -> int {  // elements with pred, over the workgroup
+      int own = 0;
+      for_elements([&](const u32x4& x, int i0) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) own += i0 + e < a.V && pred(norm(key1(elem(x, e))), i0 + e) ? 1 : 0;
+      });
+      own = wave_sum_i32(own);
+      if (lane == 0 && own) atomicAdd(&ml.count[slot], own);
+      __syncthreads();
+      return ml.count[slot];
+    };
+    __syncthreads();
+    if (tid == 0) ml.n = 0;
+    uint32_t T = 0;
+#pragma unroll 1
+    for (int bit = 15; bit >= 0; --bit) {
+      const int cut = (int)(T | (1u << bit)) - 32768;
+      if (count(bit, [&](int key, int) { return key >= cut; }) >= k) T |= 1u << bit;
+    }
+    const int cut = (int)T - 32768;
+    const int need = k - count(16, [&](int key, int) { return key > cut; });
+    uint32_t I = 0;  // the largest I with fewer than `need` equal elements below it: the last one taken
+    const int top_bit = 31 - __builtin_clz(a.V);
+#pragma unroll 1
+    for (int bit = top_bit; bit >= 0; --bit) {
+      const int c = (int)(I | (1u << bit));
+      if (count(17 + top_bit - bit, [&](int key, int idx) { return key == cut && idx < c; }) < need) I |= 1u << bit;
+    }
+    const int last = (int)I;
+    for_elements([&](const u32x4& x, int i0) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const int key = norm(key1(elem(x, e)));
+        if (i0 + e < a.V && (key > cut || (key == cut && i0 + e <= last))) {
+          const int pos = atomicAdd(&ml.n, 1);
+          if (pos < CAND_MAX) ml.cand[pos] = cand_key(elem(x, e), (uint32_t)(i0 + e));
         }
       }
-      if (lane == 0) put(i, best, logz);
+    });
+    __syncthreads();
+    n = k;
+  }
+  merge_row<NTH>(a, row, n, top + 32768, ml);
+}
+
+// ---- kernel 1 -------------------------------------------------------------------------------------------
+// What bounds it: the read of the logits, then per element 4.5 VALU and one LDS read of the sum (the table lookups),
+// about half of the load's time at eight waves per SIMD. The selection's share is the group maxima, about one
+// operation per element: the maximum of raw patterns (one packed operation per two elements) is the key of the largest
+// value unless every value is negative; a wave with such a group, or a NaN, forms the keys. 128 x 151936: 10.8 us
+// (3.6 TB/s; loads and maxima alone about 9), against 15.4 for a kernel that also took every piece's top 8;
+// 120 x 248320: 13 us, against 3.9 ms for one that kept sorted lists of 32 keys per thread for k > 32. Selecting per
+// workgroup of 16 pieces (thresholds exchanged over LDS between two barriers) instead of per row: 14.4 us.
+// ROW: rows of at most PW pieces, one workgroup per row, which also takes its top k.
+template <bool ROW>
+__global__ __launch_bounds__(NT1) __attribute__((amdgpu_waves_per_eu(ROW ? 4 : 8))) void topk_piece_kernel(TopkArgs a) {
+  __shared__ __attribute__((aligned(16))) unsigned char etab[ETAB_BYTES];
+  const int lane = threadIdx.x & 63;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int step = ROW ? PW : (int)gridDim.x * PW;
+  const int total = ROW ? a.npieces : a.rows * a.npieces;
+  int pid = ROW ? w : (int)blockIdx.x * PW + w;
+  int row = ROW ? (int)blockIdx.x : pid / a.npieces;
+  int piece = ROW ? w : pid - row * a.npieces;
+  const int drow = ROW ? 0 : step / a.npieces, dpiece = step - drow * a.npieces;
+  // group j of a piece: elements 512 j + 8 lane + e; past the row end a NaN of the lowest key, which adds nothing
+  auto load = [&](u32x4(&raw)[4]) {
+    const uint16_t* psrc = a.logits + (int64_t)row * a.row_stride + (int64_t)piece * PIECE;
+    const int nvalid = a.V - piece * PIECE;
+    if (nvalid >= PIECE) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) raw[j] = *reinterpret_cast<const u32x4*>(psrc + 512 * j + 8 * lane);
+    } else {
+      // a group starting before the row end is read whole (the buffer holds rows * row_stride elements, row_stride a
+      // multiple of 8)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int i0 = 512 * j + 8 * lane;
+        u32x4 x = {0xFFFFFFFFu, 0xFFFFFFFFu, 0xFFFFFFFFu, 0xFFFFFFFFu};
+        if (i0 < nvalid) x = *reinterpret_cast<const u32x4*>(psrc + i0);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          if (i0 + 2 * q >= nvalid) x[q] |= 0xFFFFu;
+          if (i0 + 2 * q + 1 >= nvalid) x[q] |= 0xFFFF0000u;
+        }
+        raw[j] = x;
+      }
     }
-    if (lane == 0 && a.out_logz) a.out_logz[row] = logz;
-    return;
+  };
+  u32x4 raw[4];
+  if (pid < total) load(raw);
+  etab_stage(etab);
+  __syncthreads();
+  while (pid < total) {
+    int gm[4];  // the largest key of the lane's row of 16 lanes, in group j
+    auto group_max = [&](bool keyed) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        uint32_t x = keyed ? keys2(raw[j][0]) : raw[j][0];
+#pragma unroll
+        for (int q = 1; q < 4; ++q) x = max2(x, keyed ? keys2(raw[j][q]) : raw[j][q]);
+        gm[j] = std::max((int)(int16_t)(x & 0xFFFFu), (int)x >> 16);
+      }
+#pragma unroll
+      for (int j = 0; j < 4; ++j) gm[j] = std::max(gm[j], (int)row_ror32<1>((uint32_t)gm[j]));
+#pragma unroll
+      for (int j = 0; j < 4; ++j) gm[j] = std::max(gm[j], (int)row_ror32<2>((uint32_t)gm[j]));
+#pragma unroll
+      for (int j = 0; j < 4; ++j) gm[j] = std::max(gm[j], (int)row_ror32<4>((uint32_t)gm[j]));
+#pragma unroll
+      for (int j = 0; j < 4; ++j) gm[j] = std::max(gm[j], (int)row_ror32<8>((uint32_t)gm[j]));
+    };
+    auto wave_of_rows = [&](int v) -> int {
+      return std::max(std::max(__builtin_amdgcn_readlane(v, 0), __builtin_amdgcn_readlane(v, 16)),
+                      std::max(__builtin_amdgcn_readlane(v, 32), __builtin_amdgcn_readlane(v, 48)));
+    };
+    group_max(false);
+    const int wmax = wave_of_rows(std::max(std::max(gm[0], gm[1]), std::max(gm[2], gm[3])));
+    float m = __uint_as_float((uint32_t)wmax << 16);
+    const bool neg = std::min(std::min(gm[0], gm[1]), std::min(gm[2], gm[3])) < 0;
+    if (__builtin_amdgcn_ballot_w64(neg) != 0 || wmax > 0x7F80) {
+      // negative maxima or a NaN: from the keys, and the maximum (which leaves NaNs out) from the values
+      group_max(true);
+      float x = -INFINITY;
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          x = fmaxf(x, fmaxf(__uint_as_float(raw[j][q] << 16), __uint_as_float(raw[j][q] & 0xFFFF0000u)));
+      m = wave_max_dpp(x);
+    }
+    const int64_t at = (int64_t)row * a.npieces + piece;
+    if (a.k > 0) {
+      if (a.ng == 16) {
+        // lane row r has the maxima of groups 4 j + r: a 4 x 4 transpose over the rows, then it has those of 4 r + j
+        auto swap16 = [](int& x, int& y) {
+          const auto p = __builtin_amdgcn_permlane16_swap((uint32_t)x, (uint32_t)y, false, false);
+          x = (int)p[0];
+          y = (int)p[1];
+        };
+        auto swap32 = [](int& x, int& y) {
+          const auto p = __builtin_amdgcn_permlane32_swap((uint32_t)x, (uint32_t)y, false, false);
+          x = (int)p[0];
+          y = (int)p[1];
+        };
+        swap16(gm[0], gm[1]);
+        swap16(gm[2], gm[3]);
+        swap32(gm[0], gm[2]);
+        swap32(gm[1], gm[3]);
+      } else {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) gm[j] = wave_of_rows(gm[j]);
+      }
+      const uint32_t lo = ((uint32_t)gm[0] & 0xFFFFu) | ((uint32_t)gm[1] << 16);
+      const uint32_t hi = ((uint32_t)gm[2] & 0xFFFFu) | ((uint32_t)gm[3] << 16);
+      if ((lane & 15) == 0 && lane < a.ng * 4)
+        reinterpret_cast<uint64_t*>(a.ws_g)[at * (a.ng / 4) + (lane >> 4)] = ((uint64_t)hi << 32) | lo;
+    }
+    const uint16_t* psrc = a.logits + (int64_t)row * a.row_stride + (int64_t)piece * PIECE;
+    const float ssum = wave_sum_tree(piece_lane_sum(raw, m, psrc, a.V - piece * PIECE, etab));
+    if (lane == 0) {
+      a.ws_m[at] = m;
+      a.ws_s[at] = (double)ssum;
+    }
+    if constexpr (ROW) break;
+    pid += step;
+    row += drow;
+    piece += dpiece;
+    if (piece >= a.npieces) {
+      piece -= a.npieces;
+      ++row;
+    }
+    if (pid < total) load(raw);
   }
-  uint64_t v = lane < n ? cs[lane] : 0ull;
-  int next = 64;
-  uint64_t km;
-  for (;;) {
-    const uint64_t t = wave_kth_largest64(v, k);
-    const bool keep = v != 0ull && v >= t;
-    km = __builtin_amdgcn_ballot_w64(keep);
-    if (next >= n) break;
-    const int nk = __builtin_popcountll(km);
-    if (keep) keep_buf[__builtin_amdgcn_mbcnt_hi((uint32_t)(km >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)km, 0))] = v;
-    __builtin_amdgcn_s_waitcnt(0);
-    __builtin_amdgcn_wave_barrier();
-    const int i = next + lane - nk;
-    v = lane < nk ? keep_buf[lane] : (i < n ? cs[i] : 0ull);
-    __builtin_amdgcn_s_waitcnt(0);
-    __builtin_amdgcn_wave_barrier();
-    next += 64 - nk;
+  if constexpr (ROW) {
+    __shared__ MergeLds ml;
+    __shared__ double terms[PW + 2];
+    __syncthreads();  // the row's maxima, sums and group keys are written
+    row_topk<NT1>(a, blockIdx.x, ml, terms);
   }
-  // output position of a kept key = number of kept keys larger than it
-  const bool keep = (km >> lane) & 1ull;
-  const int nk = __builtin_popcountll(km);
-  int rank = 0;
-  uint64_t rest = km;
-  while (rest) {
-    const int j = (int)__builtin_ctzll(rest);
-    rest &= rest - 1;
-    const uint64_t vj = ((uint64_t)(uint32_t)__builtin_amdgcn_readlane((uint32_t)(v >> 32), j) << 32) |
-                        (uint32_t)__builtin_amdgcn_readlane((uint32_t)v, j);
-    rank += vj > v ? 1 : 0;
-  }
-  if (keep) put(rank, v, logz);
-  if (lane >= nk && lane < k) put(lane, 0ull, logz);
-  if (lane == 0 && a.out_logz) a.out_logz[row] = logz;
+}
+
+// ---- kernel 2 -------------------------------------------------------------------------------------------
+template <int NTH>
+__global__ __launch_bounds__(NTH) void topk_row_kernel(TopkArgs a) {
+  extern __shared__ __align__(16) unsigned char dyn[];  // npieces + 1 doubles
+  __shared__ MergeLds ml;
+  row_topk<NTH>(a, blockIdx.x, ml, reinterpret_cast<double*>(dyn));
 }
 
 }  // namespace
 
 extern "C" int64_t mfd_topk_logz_workspace_bytes(int rows, int V, int k) {
   const int64_t npieces = ((int64_t)V + PIECE - 1) / PIECE;
-  // per piece: m (4 bytes), S (8) and up to k candidate keys (the k > 32 kernel keeps k per 4 pieces)
+  // per piece: m (4 bytes), S (8) and room for k candidate keys
   return (int64_t)rows * npieces * (4 + 8 + 8 * (int64_t)(k > 0 ? k : 1)) + 64;
 }
 
@@ -877,10 +854,9 @@ static int topk_logz_impl(const uint16_t* logits, int rows, int V, int64_t row_s
     return mfd_set_error(MFD_ERR_INVALID_ARG, "mfd_topk_logz: bad sizes rows=%d V=%d k=%d", rows, V, k);
   if (k > KMAX) return mfd_set_error(MFD_ERR_UNSUPPORTED, "mfd_topk_logz: k=%d > %d", k, KMAX);
   const int npieces = (V + PIECE - 1) / PIECE;
-  const int nchunks = (V + CHUNK - 1) / CHUNK;
   const int kk = k > 0 ? k : 1;
-  const int nlists = kk <= 32 ? npieces : nchunks;
-  if ((int64_t)nlists * kk > FINAL_CAND)
+  const int nlists = kk <= 32 ? npieces : (V + 8191) / 8192;
+  if ((int64_t)nlists * kk > MERGE_MAX)
     return mfd_set_error(MFD_ERR_UNSUPPORTED, "mfd_topk_logz: V=%d with k=%d exceeds the merge capacity", V, k);
   if (row_stride < V || (row_stride % 8) != 0 || (reinterpret_cast<uintptr_t>(logits) % 16) != 0)
     return mfd_set_error(MFD_ERR_UNSUPPORTED, "mfd_topk_logz: rows must be 16-byte aligned (stride %lld)",
@@ -892,44 +868,33 @@ static int topk_logz_impl(const uint16_t* logits, int rows, int V, int64_t row_s
   if (!workspace || workspace_bytes < need)
     return mfd_set_error(MFD_ERR_INVALID_ARG, "mfd_topk_logz: workspace of %lld bytes needed", (long long)need);
   char* ws = static_cast<char*>(workspace);
-  uint64_t* cand = reinterpret_cast<uint64_t*>(ws);
   double* s = reinterpret_cast<double*>(ws + (int64_t)rows * npieces * kk * 8);
   float* m = reinterpret_cast<float*>(ws + (int64_t)rows * npieces * (kk * 8 + 8));
-  ChunkArgs ca{logits, row_stride, rows, V, kk, npieces, nchunks, m, s, cand};
-  FinalArgs fa{rows, k, npieces, nlists, m, s, cand, out_logp, out_ids, ids_int64, out_logz, vocab_ids};
+  // the group keys take up to 32 of the 8 max(k, 1) bytes per piece
+  const int ng = kk >= 4 ? 16 : 4;
+  TopkArgs a{logits, row_stride, rows, V, k, npieces, ng, m, s, reinterpret_cast<int16_t*>(ws), out_logp, out_ids, ids_int64,
+             out_logz, vocab_ids};
   hipStream_t st = static_cast<hipStream_t>(stream);
-  if (kk <= 32) {
-    // one wave per piece while that fits two workgroups per CU; beyond, the waves loop over pieces
-    const int64_t total = (int64_t)rows * npieces;
-    if (k > 0 && k <= 8 && npieces <= PW) {
-      // rows of at most PW pieces: one workgroup per row, which also merges it
-      hipLaunchKernelGGL((topk_piece_kernel<8, true>), dim3((unsigned)rows), dim3(PW * 64), 0, st, ca, fa);
-      MFD_CHECK_LAUNCH();
-      return MFD_OK;
-    }
-    const dim3 grid((unsigned)std::min<int64_t>((total + PW - 1) / PW, 2 * (int64_t)mfd_num_cus()));
-    if (kk <= 8)
-      hipLaunchKernelGGL((topk_piece_kernel<8, false>), grid, dim3(PW * 64), 0, st, ca, fa);
-    else if (kk <= 16)
-      hipLaunchKernelGGL((topk_piece_kernel<16, false>), grid, dim3(PW * 64), 0, st, ca, fa);
-    else
-      hipLaunchKernelGGL((topk_piece_kernel<32, false>), grid, dim3(PW * 64), 0, st, ca, fa);
-    MFD_CHECK_LAUNCH();
-    {
-      const int rc = mfd_set_max_lds(reinterpret_cast<const void*>(&topk_small_final_kernel), 160 * 1024);
-      if (rc != MFD_OK) return rc;
-    }
-    const int ncand = nlists * k;
-    const size_t smem = (size_t)(npieces + 64 + (ncand <= FINAL_STAGE ? ncand : 0)) * sizeof(double);
-    hipLaunchKernelGGL(topk_small_final_kernel, dim3(rows), dim3(64), smem, st, fa);
+  if (npieces <= PW) {
+    hipLaunchKernelGGL(topk_piece_kernel<true>, dim3((unsigned)rows), dim3(NT1), 0, st, a);
     MFD_CHECK_LAUNCH();
     return MFD_OK;
   }
-  const dim3 grid((unsigned)((int64_t)rows * nchunks));
-  // k > 32: a thread's 32-entry list keeps all of its elements
-  hipLaunchKernelGGL(topk_logz_chunk_kernel<PER>, grid, dim3(NT), 0, st, ca);
+  // one wave per piece while that fits two workgroups per CU; beyond, the waves take further pieces in turn
+  const int64_t total = (int64_t)rows * npieces;
+  const dim3 grid((unsigned)std::min<int64_t>((total + PW - 1) / PW, 2 * (int64_t)mfd_num_cus()));
+  hipLaunchKernelGGL(topk_piece_kernel<false>, grid, dim3(NT1), 0, st, a);
   MFD_CHECK_LAUNCH();
-  hipLaunchKernelGGL(topk_logz_final_kernel, dim3(rows), dim3(64), 0, st, fa);
+  const size_t smem = (size_t)((npieces + 3) & ~1) * sizeof(double);
+  if (kk <= 32) {
+    const int rc = mfd_set_max_lds(reinterpret_cast<const void*>(&topk_row_kernel<256>), 128 * 1024);
+    if (rc != MFD_OK) return rc;
+    hipLaunchKernelGGL(topk_row_kernel<256>, dim3(rows), dim3(256), smem, st, a);
+  } else {
+    const int rc = mfd_set_max_lds(reinterpret_cast<const void*>(&topk_row_kernel<1024>), 128 * 1024);
+    if (rc != MFD_OK) return rc;
+    hipLaunchKernelGGL(topk_row_kernel<1024>, dim3(rows), dim3(1024), smem, st, a);
+  }
   MFD_CHECK_LAUNCH();
   return MFD_OK;
 }

@@ -53,6 +53,49 @@ def test_topk_logz_bit_exact(kind, rows, V, k):
     np.testing.assert_array_equal(logp.cpu().numpy().view(np.uint32), lp_ref.view(np.uint32))
 
 
+def _edge_logits(kind, rows, V, k, seed):
+    """Rows where a selection by group maxima can go wrong: all values equal, all negative, fewer than k unmasked
+    values among the lowest finite value or -inf, the top values next to each other in one group of 128, zeros of both
+    signs at the k-th place, and values over the whole exponent range."""
+    g = torch.Generator().manual_seed(seed)
+    x = torch.randn(rows, V, generator=g)
+    if kind == "equal":
+        x = torch.full((rows, V), 1.5)
+    elif kind == "negative":
+        x = -x.abs() * 4 - 1
+    elif kind in ("masked_low", "masked_inf"):
+        low = torch.finfo(torch.bfloat16).min if kind == "masked_low" else float("-inf")
+        keep = torch.rand(rows, V, generator=g) < (k // 2) / V
+        x = torch.where(keep, x, torch.tensor(low))
+    elif kind == "adjacent":
+        at = V // 3
+        x[:, at:at + 2 * k] += 20 + torch.arange(min(2 * k, V - at)) / 16
+    elif kind == "zeros":
+        x = torch.where(torch.rand(rows, V, generator=g) < 0.3, torch.zeros(()), -x.abs())
+        x = torch.where(torch.rand(rows, V, generator=g) < 0.5, x, -0.0 * torch.ones(()))
+    elif kind == "range":
+        x = x * torch.exp2(torch.randint(-60, 7, (rows, V), generator=g).float())
+    return x.to(torch.bfloat16)
+
+
+@pytest.mark.parametrize("kind", ["equal", "negative", "masked_low", "masked_inf", "adjacent", "zeros", "range"])
+@pytest.mark.parametrize("rows,V,k", [(3, 2047, 256), (2, 2049, 33), (5, 32768, 8), (3, 32769, 256), (3, 40001, 3),
+                                      (2, 70000, 32), (2, 131073, 64), (1, 248320, 256)])
+def test_topk_logz_selection_edges(kind, rows, V, k):
+    """Bit-exact like every other row: one and several launches per row, ends of pieces and groups, both group sizes,
+    more candidates than the merge holds."""
+    import tree_logits
+
+    x = _edge_logits(kind, rows, V, k, seed=V + k)
+    print(f"case: topk_logz edges {kind} rows={rows} V={V} k={k}", flush=True)
+    logp, ids, logz = tree_logits.topk_logz(x.cuda(), k, with_logz=True)
+    torch.cuda.synchronize()
+    lp_ref, ids_ref, lz_ref = B.top_candidates(x, k)
+    np.testing.assert_array_equal(ids.cpu().numpy(), ids_ref)
+    np.testing.assert_array_equal(logz.cpu().numpy().view(np.uint32), lz_ref.view(np.uint32))
+    np.testing.assert_array_equal(logp.cpu().numpy().view(np.uint32), lp_ref.view(np.uint32))
+
+
 def test_row_logsumexp_and_top_candidates_api():
     import tree_logits
 
