@@ -350,6 +350,34 @@ def test_tree_gates(sizes, H, dtype):
     np.testing.assert_allclose(G.cpu().numpy(), G_ref, rtol=0, atol=1e-5 * np.abs(G_ref).max())
 
 
+@pytest.mark.parametrize("case", ["deep", "long", "many"])
+def test_tree_gates_deep_long_and_many_requests(case):
+    """Paths of more than 32 nodes, ancestors more than 1024 nodes back, more than 256 requests; a head count that no
+    workgroup divides. The parents need no depth limit here."""
+    import tree_gdn_kernel
+
+    rng = np.random.default_rng(5)
+    H = 5
+    if case == "deep":  # a chain of 70, then nodes anywhere below it
+        trees = [np.concatenate([np.arange(-1, 69), rng.integers(0, 70, 30)])]
+    elif case == "long":  # 1400 nodes whose parents are among the first 40
+        trees = [np.array([-1, 0, 1]), np.concatenate([np.arange(-1, 39), rng.integers(0, 40, 1360)])]
+    else:
+        trees = [np.array([-1, 0, 0, 2][: 1 + i % 4]) for i in range(300)]
+    parents = np.concatenate(trees).astype(np.int32)
+    cu = np.concatenate([[0], np.cumsum([len(t) for t in trees])]).astype(np.int32)
+    g = torch.Generator().manual_seed(3)
+    a, b = torch.randn(len(parents), H, generator=g), torch.randn(len(parents), H, generator=g)
+    A_log, dt = torch.randn(H, generator=g) * 0.5, torch.randn(H, generator=g)
+    G, beta = tree_gdn_kernel.tree_gates(a.cuda(), b.cuda(), A_log.cuda(), dt.cuda(), parents=torch.from_numpy(parents).cuda(),
+                                         cu_nodes=torch.from_numpy(cu).cuda())
+    torch.cuda.synchronize()
+    G_ref, beta_ref = _gates_ref(a, b, A_log, dt, parents, cu, torch.float32)
+    np.testing.assert_allclose(beta.cpu().numpy(), beta_ref, rtol=0, atol=1e-6)
+    # fp32 sums of at most 70 terms of one sign
+    np.testing.assert_allclose(G.cpu().numpy(), G_ref, rtol=0, atol=1e-5 * np.abs(G_ref).max())
+
+
 def test_tree_gates_anc8_and_into_tree_gdn():
     """Single tree given by its ancestor matrix (the HF TreeContext form); the gates then feed tree_gdn,
     which must match the oracle fed with the oracle's gates."""
