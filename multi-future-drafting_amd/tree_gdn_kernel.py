@@ -76,7 +76,7 @@ def tree_gdn(q, k, v, g_cum, beta, s0, anc8, block_t: int = 64, block_v: int = 3
     q, k, v = q.contiguous(), k.contiguous(), v.contiguous()
     g_cum, beta = g_cum.contiguous().float(), beta.contiguous().float()
     s0 = s0.contiguous().float()
-    anc8 = anc8.contiguous().to(torch.int8)
+    anc8 = mfd_hip.as_dtype(anc8.contiguous(), torch.int8)
     u = torch.empty(N, H, D, dtype=torch.float32, device=k.device)
     o = torch.empty(N, H, D, dtype=torch.float32, device=k.device)
     ws = _workspace(1, N, HK, N, False, k.device)
@@ -210,16 +210,15 @@ def tree_gates(a: torch.Tensor, b: torch.Tensor, A_log: torch.Tensor, dt_bias: t
     if a.stride(1) != 1:
         a, b = a.contiguous(), b.contiguous()
     N, H = a.shape
-    A_log = A_log.reshape(H).float().contiguous()
-    dt_bias = dt_bias.reshape(H).float().contiguous()
+    A_log, dt_bias = ((t if t.shape == (H,) else t.reshape(H)).float().contiguous() for t in (A_log, dt_bias))
     if parents is None and anc8 is None:
         raise ValueError("parents or anc8 required")
     if parents is not None:
-        parents = parents.to(torch.int32).contiguous()
+        parents = mfd_hip.as_dtype(parents, torch.int32).contiguous()
     if anc8 is not None and parents is None:
-        anc8 = anc8.to(torch.int8).contiguous()
+        anc8 = mfd_hip.as_dtype(anc8, torch.int8).contiguous()
     R = 1 if cu_nodes is None else cu_nodes.numel() - 1
-    cu = None if cu_nodes is None else cu_nodes.to(torch.int32).contiguous()
+    cu = None if cu_nodes is None else mfd_hip.as_dtype(cu_nodes, torch.int32).contiguous()
     g_cum = torch.empty(N, H, dtype=torch.float32, device=a.device)
     beta = torch.empty(N, H, dtype=torch.float32, device=a.device)
     mfd_hip.call("mfd_tree_gates", a.data_ptr(), b.data_ptr(), 1 if a.dtype == torch.bfloat16 else 0, a.stride(0),
@@ -264,11 +263,11 @@ def tree_prep(x, conv_state, conv_index, conv_w, num_k_heads: int, num_v_heads: 
     R = 1 if cu_nodes is None else cu_nodes.numel() - 1
     if conv_state.dim() == 3 and conv_state.shape[0] != R:
         raise ValueError("conv_state [R, conv_dim, KC] must match cu_nodes")
-    x = x.to(torch.bfloat16)
+    x = mfd_hip.as_dtype(x, torch.bfloat16)
     if x.stride(1) != 1 or x.stride(0) % 8 or x.data_ptr() % 16:
         x = x.contiguous()
-    conv_state = conv_state.to(torch.bfloat16).contiguous()
-    conv_w = conv_w.to(torch.bfloat16).contiguous()
+    conv_state = mfd_hip.as_dtype(conv_state, torch.bfloat16).contiguous()
+    conv_w = mfd_hip.as_dtype(conv_w, torch.bfloat16).contiguous()
     q = torch.empty(n, HK, D, dtype=torch.bfloat16, device=x.device)
     k = torch.empty_like(q)
     v = torch.empty(n, H, D, dtype=torch.bfloat16, device=x.device)
@@ -296,7 +295,9 @@ def gdn_commit(recurrent, u, k, g_cum, path, conv=None, x=None, conv_index=None,
     dev = u.device
     if not torch.is_tensor(path):
         path = torch.tensor(list(path), dtype=torch.int32)
-    path = path.to(device=dev, dtype=torch.int32).contiguous()
+    if path.device != dev or path.dtype != torch.int32:
+        path = path.to(device=dev, dtype=torch.int32)
+    path = path.contiguous()
     mfd_hip.require_cuda(recurrent, u, k, g_cum, conv, x, conv_index)
     L, n, H, D = u.shape
     HK = k.shape[2]
@@ -308,7 +309,7 @@ def gdn_commit(recurrent, u, k, g_cum, path, conv=None, x=None, conv_index=None,
     if k.shape != (L, n, HK, D) or g_cum.shape != (L, n, H):
         raise ValueError("k must be [L, n, HK, D] and g_cum [L, n, H]")
     u = u.float().contiguous()
-    k = k.to(torch.bfloat16).contiguous()
+    k = mfd_hip.as_dtype(k, torch.bfloat16).contiguous()
     g_cum = g_cum.float().contiguous()
     p = path.numel()
     cptr, xptr, ciptr, CD, KC, c_lst, x_lst, x_rst = None, None, None, 0, 0, 0, 0, 0
@@ -319,12 +320,12 @@ def gdn_commit(recurrent, u, k, g_cum, path, conv=None, x=None, conv_index=None,
         if cv.shape[0] != L:
             raise ValueError("conv must be contiguous bfloat16 [L, CD, KC] (or [L, 1, CD, KC])")
         CD, KC = cv.shape[1], cv.shape[2]
-        x = _stack(x).to(torch.bfloat16)
+        x = mfd_hip.as_dtype(_stack(x), torch.bfloat16)
         if x.shape != (L, n, CD) or x.stride(2) != 1:
             x = x.contiguous()
         if conv_index is None or conv_index.shape != (n, KC):
             raise ValueError("conv_index [n, KC] is required with conv")
-        cptr, xptr, ciptr = cv.data_ptr(), x.data_ptr(), conv_index.to(torch.int32).contiguous().data_ptr()
+        cptr, xptr, ciptr = cv.data_ptr(), x.data_ptr(), mfd_hip.as_dtype(conv_index, torch.int32).contiguous().data_ptr()
         c_lst, x_lst, x_rst = CD * KC, x.stride(0), x.stride(1)
     mfd_hip.call("mfd_gdn_commit", state.data_ptr(), H * D * D, u.data_ptr(), n * H * D, k.data_ptr(), n * HK * D,
                  g_cum.data_ptr(), n * H, path.data_ptr(), p, L, n, HK, H, D, cptr, c_lst, xptr, x_lst, x_rst,
