@@ -68,34 +68,36 @@ __device__ __forceinline__ void stage_lds(const T* src, int32_t* dst, int n, int
   }
 }
 
-// Outputs of request b: tree[b] = tokens, depths, parents of width budget + 1 (index 0 = root; tail entries
-// 0, 0, -1), counts[b], and the ancestor-or-self matrix when requested.
-__device__ void write_tree(const BuildArgs& a, int b, int lane, int count, const int32_t* npar, const int32_t* ntok,
-                           const int32_t* ndep) {
+// Zeroes the ancestor matrix of request b, by threads t = 0 .. n - 1 (n a multiple of 64).
+__device__ __forceinline__ void zero_anc8(const BuildArgs& a, int b, int t, int n) {
+  const int W = a.budget + 1;
+  int8_t* vis = a.anc8 + (int64_t)b * W * W;
+  const int64_t WW = (int64_t)W * W;
+  // bytes up to the first 16-byte boundary, 16-byte stores, then the remaining bytes
+  const int64_t head = min(WW, (int64_t)((16 - (reinterpret_cast<uintptr_t>(vis) & 15)) & 15));
+  const int64_t nvec = (WW - head) / 16;
+  for (int64_t f = t; f < head; f += n) vis[f] = 0;
+  uint4* vv = reinterpret_cast<uint4*>(vis + head);
+  for (int64_t f = t; f < nvec; f += n) vv[f] = make_uint4(0u, 0u, 0u, 0u);
+  for (int64_t f = head + nvec * 16 + t; f < WW; f += n) vis[f] = 0;
+}
+// Outputs of request b, by threads t = 0 .. n - 1: tree[b] = tokens, depths, parents of width budget + 1 (index 0 =
+// root; tail entries 0, 0, -1), counts[b], and the ancestor-or-self entries of rows 0 .. count of the (zeroed, and
+// visibly so) matrix when requested, one row per thread, walking up the parents.
+__device__ __forceinline__ void write_tree(const BuildArgs& a, int b, int t0, int n, int count, const int32_t* npar,
+                                           const int32_t* ntok, const int32_t* ndep) {
   const int W = a.budget + 1;
   int64_t* t = a.tree + (int64_t)b * 3 * W;
-  for (int i = lane; i < W; i += WAVE) {
+  for (int i = t0; i < W; i += n) {
     const bool used = i <= count;
     t[i] = (used && i > 0) ? (int64_t)ntok[i] : 0;
     t[W + i] = used ? (int64_t)ndep[i] : 0;
     t[2 * W + i] = used ? (int64_t)npar[i] : -1;
   }
-  if (lane == 0) a.counts[b] = count;
+  if (t0 == 0) a.counts[b] = count;
   if (a.anc8) {
     int8_t* vis = a.anc8 + (int64_t)b * W * W;
-    // zero the matrix with wave-coalesced stores, make those stores visible to the wave, then set the
-    // ancestor-or-self entries of rows 0..count (one row per lane, walking up the parents)
-    const int64_t WW = (int64_t)W * W;
-    // bytes up to the first 16-byte boundary, 16-byte stores, then the remaining bytes
-    const int64_t head = min(WW, (int64_t)((16 - (reinterpret_cast<uintptr_t>(vis) & 15)) & 15));
-    const int64_t nvec = (WW - head) / 16;
-    for (int64_t f = lane; f < head; f += WAVE) vis[f] = 0;
-    uint4* vv = reinterpret_cast<uint4*>(vis + head);
-    for (int64_t f = lane; f < nvec; f += WAVE) vv[f] = make_uint4(0u, 0u, 0u, 0u);
-    for (int64_t f = head + nvec * 16 + lane; f < WW; f += WAVE) vis[f] = 0;
-    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
-    __builtin_amdgcn_wave_barrier();
-    for (int i = lane; i <= count; i += WAVE) {
+    for (int i = t0; i <= count; i += n) {
       int8_t* row = vis + (int64_t)i * W;
       int cur = i;
       while (cur >= 0) {
@@ -106,23 +108,23 @@ __device__ void write_tree(const BuildArgs& a, int b, int lane, int count, const
   }
 }
 
-// (token, log-prob bits) records of the request's top lists, staged by one wave: batches of 16 entries per
-// lane, all loads issued before the first one is used (int64 ids keep their low 32 bits)
-template <typename T>
+// (token, log-prob bits) records of the request's top lists, staged by NT threads: batches of 8 entries per
+// thread, all loads issued before the first one is used (int64 ids keep their low 32 bits)
+template <int NT, typename T>
 __device__ __forceinline__ void stage_records(const float* lp, const T* ids, int2* rec, int n, int lane) {
-  constexpr int SB = 16;
-  for (int i0 = 0; i0 < n; i0 += SB * WAVE) {
+  constexpr int SB = 8;
+  for (int i0 = 0; i0 < n; i0 += SB * NT) {
     float v[SB];
     int32_t t[SB];
 #pragma unroll
     for (int u = 0; u < SB; ++u) {
-      const int i = min(i0 + u * WAVE + lane, n - 1);
+      const int i = min(i0 + u * NT + lane, n - 1);
       v[u] = lp[i];
       t[u] = (int32_t)ids[i];
     }
 #pragma unroll
     for (int u = 0; u < SB; ++u)
-      if (i0 + u * WAVE + lane < n) rec[i0 + u * WAVE + lane] = make_int2(t[u], __float_as_int(v[u]));
+      if (i0 + u * NT + lane < n) rec[i0 + u * NT + lane] = make_int2(t[u], __float_as_int(v[u]));
   }
 }
 
@@ -136,10 +138,19 @@ __device__ __forceinline__ float readlane_f32(float v, int l) {
 }
 
 // Frontier rows held in registers: slot s belongs to lane s % 64, row s / 64; rows below RR are registers,
-// rows from RR on (large or heavily merged frontiers) live in LDS.
-constexpr int RR = 2;
+// rows from RR on (heavily merged frontiers) live in LDS. A pop opens at most one slot, so 2 rows hold the frontier
+// of 64 nodes and 5 that of 256 (and K modes) unless modes keep popping each other's prefixes.
+constexpr int frontier_rows(int nr) { return nr >= 4 ? 6 : nr == 2 ? 3 : 2; }
 constexpr int BMAX = 64;  // entries one batch pops at most (one per lane)
-constexpr int BMIN = 6;   // frontier heads below sigma from which a batch is tried
+constexpr int BMIN = 3;   // candidates from which a batch is taken
+constexpr int FEW = 6;    // lists up to which several lanes share one
+constexpr int MNT = 256;  // threads of build_mixture_kernel: wave 0 builds, the others stage and write
+// set bits of m below this lane
+__device__ __forceinline__ int lanes_below(uint64_t m) {
+  return (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0));
+}
+// Orders a wave's LDS accesses for the compiler and waits for them (the wave's own are processed in order).
+__device__ __forceinline__ void wave_sync() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
 
 constexpr uint64_t HEMPTY = ~0ull;
 __device__ __forceinline__ uint32_t hash_pt(int parent, int token) {
@@ -164,27 +175,36 @@ __device__ __forceinline__ bool pair_lt(uint32_t ka, uint32_t fa, uint32_t kb, u
 // sibling adds lp_{r+1} - lp_r <= 0, up to an fp64 rounding that is checked), so the pop order is the
 // (key bits, fields) order of all entries. With sigma = the smallest child key over the frontier, every
 // frontier entry with key < sigma, together with the frontier minimum f1, pops before anything a pop can
-// generate; the siblings of a head below sigma are such entries too. When at least BMIN heads are below
-// sigma, one step pops that whole prefix: the candidates (heads, and their siblings while below sigma; at
-// most 64) are ordered by (key, fields), all their parents being known nodes, so the order is the heap's,
-// ties included; the batch is cut after an entry whose next sibling would order before the next batch entry
-// (an fp64 rounding that put that sibling's key below its elder's: the walk stops before such a sibling) and
-// after the pop that creates node number budget. Otherwise the step pops f1 alone.
+// generate; the siblings of a head below sigma are such entries too. A step gives each of the nl lists with a head below
+// sigma (and f1's) 64 / nl lanes, lane t of a list forming its t-th next sibling (many lists: one lane each, which
+// forms a few), and pops every one of them below sigma and below the first sibling that no lane formed, and of those
+// the smallest 64; with fewer than BMIN it pops f1 alone. The candidates are
+// ordered by (key, fields), all their parents being known nodes, so the order is the heap's, ties included; the batch
+// is cut after an entry whose next sibling would order before the next batch entry (an fp64 rounding that put that
+// sibling's key below its elder's: a list's candidates end before such a sibling) and after the pop that creates
+// node number budget.
 //
 // LDS layout (dynamic): slot logw f64 [cap], slot key u32 [cap], slot fields u32 [cap], slot child key
 // u32 [cap], slot last-popped rank i32 [cap] (rows >= RR always; register rows are copied in for a batch),
-// candidate logw f64 [64], key / fields / slot u32 [64], records (token, lp bits) [K L k], prior f32 [16],
+// candidate logw f64 [64], (key, fields) u64 [64], slot u32 [64], records (token, lp bits) [K L k], prior f32 [16],
 // node parent / token / depth i32 [budget + 1], counter i32 [4].
 // NR = register slots per lane of the node table (64 NR >= budget).
 //
+// What bounds it: the issue rate of one wave, 7-10 thousand cycles per batch step (enumeration 2.3, ranking 1-2, nodes
+// and lists 3) against 2-2.8 thousand per sequential pop, so a batch pays from 3 entries on. Logits of randn * 3, one
+// request, with the candidates' entry copies and the ancestor matrix, against batches that took only lists of at most 8
+// entries and frontiers of 128 slots: K 8, L 16, k 8, B 64 17.4 -> 14.5 us; K 8, k 64, B 64 66 -> 25; K 1, k 64, B 64
+// 57 -> 27; K 8, k 8, B 256 207 -> 33; K 4, k 256, B 256 287 -> 73; K 1, k 256, B 256 282 -> 167.
 // A sequential pop needs no LDS round trip: every lane keeps its best slot's key, fields, row and logw in
 // registers, and after each pop every lane prefetches the records its best entry will need if popped.
 template <int NR>
-__global__ __launch_bounds__(WAVE) void build_mixture_kernel(BuildArgs a) {
+__global__ __launch_bounds__(MNT) void build_mixture_kernel(BuildArgs a) {
 #pragma clang fp contract(off)
   extern __shared__ __align__(16) unsigned char smem[];
+  constexpr int RR = frontier_rows(NR);
   const int b = blockIdx.x;
-  const int lane = threadIdx.x;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int K = a.K, L = a.L, kk = a.k, cap = a.cap, budget = a.budget;
   const int nlp = K * L * kk;
   const int HS = a.hsize;
@@ -197,9 +217,8 @@ __global__ __launch_bounds__(WAVE) void build_mixture_kernel(BuildArgs a) {
   int32_t* fmax = reinterpret_cast<int32_t*>(fck + cap);
   int32_t* hid = fmax + cap;
   int32_t* hmin = hid + HS;
-  uint32_t* ck = reinterpret_cast<uint32_t*>(hmin + HS);
-  uint32_t* cf = ck + BMAX;
-  int32_t* cs = reinterpret_cast<int32_t*>(cf + BMAX);
+  uint64_t* c64 = reinterpret_cast<uint64_t*>(hmin + HS);  // a batch's candidates: key in the upper, fields in the lower half
+  int32_t* cs = reinterpret_cast<int32_t*>(c64 + BMAX);
   int2* rec = reinterpret_cast<int2*>(cs + BMAX);
   float* sprior = reinterpret_cast<float*>(rec + nlp);
   int32_t* npar = reinterpret_cast<int32_t*>(sprior + 16);
@@ -209,14 +228,24 @@ __global__ __launch_bounds__(WAVE) void build_mixture_kernel(BuildArgs a) {
 
   const float* lpb = a.lp + (int64_t)b * nlp;
   if (a.ids_int64)
-    stage_records(lpb, static_cast<const int64_t*>(a.ids) + (int64_t)b * nlp, rec, nlp, lane);
+    stage_records<MNT>(lpb, static_cast<const int64_t*>(a.ids) + (int64_t)b * nlp, rec, nlp, (int)threadIdx.x);
   else
-    stage_records(lpb, static_cast<const int32_t*>(a.ids) + (int64_t)b * nlp, rec, nlp, lane);
-  for (int s = lane; s < cap; s += WAVE) fmax[s] = -1;
-  for (int h = lane; h < HS; h += WAVE) {
+    stage_records<MNT>(lpb, static_cast<const int32_t*>(a.ids) + (int64_t)b * nlp, rec, nlp, (int)threadIdx.x);
+  for (int s = threadIdx.x; s < cap; s += MNT) fmax[s] = -1;
+  for (int h = threadIdx.x; h < HS; h += MNT) {
     hkey[h] = HEMPTY;
     hid[h] = -1;
     hmin[h] = 0x7FFFFFFF;
+  }
+  if (threadIdx.x < K) sprior[threadIdx.x] = a.prior ? a.prior[(int64_t)b * K + threadIdx.x] : 0.f;
+  __syncthreads();
+  if (wave != 0) {
+    // the other waves zero the matrix meanwhile and wait for the tree; the last barrier makes the zeros visible
+    if (a.anc8) zero_anc8(a, b, (int)threadIdx.x - WAVE, MNT - WAVE);
+    __builtin_amdgcn_s_waitcnt(0);
+    __syncthreads();
+    write_tree(a, b, (int)threadIdx.x, MNT, scnt[0], npar, ntok, ndep);
+    return;
   }
   auto lp_at = [&](int m, int row, int r) __attribute__((always_inline)) {
     return __int_as_float(rec[(m * L + row) * kk + r].y);
@@ -236,9 +265,6 @@ __global__ __launch_bounds__(WAVE) void build_mixture_kernel(BuildArgs a) {
   uint32_t lhi = NONE, llo = NONE, lcm = NONE;
   int lrow = 0;
   double lbw = 0.0;
-  if (lane < K) sprior[lane] = a.prior ? a.prior[(int64_t)b * K + lane] : 0.f;
-  __builtin_amdgcn_s_waitcnt(0);
-  __syncthreads();
   // seed: one entry per mode (rank 0 at depth 1 under the root) in slot m, which lane m owns (K <= 16)
   if (lane < K) {
     const float pr = sprior[lane];
@@ -310,155 +336,233 @@ __global__ __launch_bounds__(WAVE) void build_mixture_kernel(BuildArgs a) {
   };
   prefetch();
 
-  int count = 0, tail = K, alive = K, hashed = 0, next_check = 0, gap = 2;
+  int count = 0, tail = K, alive = K, hashed = 0, next_check = 0, gap = 1;
   bool overflow = false;
   // Batch step: pops the prefix of the frontier order below sigma at once (see above). Returns false, with
-  // nothing changed, when the candidates exceed 64 or a list has more than WALK of them.
+  // nothing changed, when fewer than BMIN entries are certain or more than 64 lists qualify.
   auto batch_step = [&](uint32_t f1, uint32_t mh, uint32_t sigma) -> bool {
-    constexpr int WALK = 8;
     if (tail > RR * WAVE) return false;
-    // register rows to LDS; the nodes made by sequential pops since the last batch into the hash table
+    // more than 64 lists below sigma: a lower one
+    auto heads_below = [&](uint32_t key) -> int {
+      int n = 0;
+#pragma unroll
+      for (int rr = 0; rr < RR; ++rr)
+        if (rr * WAVE < tail) n += __builtin_popcountll(__builtin_amdgcn_ballot_w64(khi[rr] < key));
+      return n;
+    };
+    if (heads_below(sigma) > BMAX) {
+      uint32_t lo = mh, hi = sigma;  // at most 63 heads below lo (none), more than 64 below hi
+      for (int it = 0; it < 16; ++it) {
+        const uint32_t mid = lo + (hi - lo) / 2;
+        const int n = heads_below(mid);
+        if (n > BMAX) hi = mid; else lo = mid;
+        if (n <= BMAX && n > BMAX / 2) break;
+      }
+      sigma = lo;
+    }
+    // the lists with a head below sigma (f1's in any case): their slots in cs, their heads to LDS
+    int nl = 0;
+    bool ql[RR];
 #pragma unroll
     for (int rr = 0; rr < RR; ++rr) {
-      const int s = rr * WAVE + lane;
-      if (s < tail) {
-        fhi[s] = khi[rr];
-        flo[s] = klo[rr];
-        fck[s] = kck[rr];
-        flogw[s] = klw[rr];
-      }
-    }
-#pragma unroll
-    for (int r = 0; r < NR; ++r) {
-      const int id = 64 * r + lane + 1;
-      if (id > hashed && id <= count) {
-        const uint64_t key64 = ((uint64_t)(uint32_t)rpar[r] << 32) | (uint32_t)rtok[r];
-        int slot = (int)(hash_pt(rpar[r], rtok[r]) & (uint32_t)(HS - 1));
-        for (int probe = 0; probe < HS; ++probe) {
-          const uint64_t old = atomicCAS(reinterpret_cast<unsigned long long*>(&hkey[slot]),
-                                         (unsigned long long)HEMPTY, (unsigned long long)key64);
-          if (old == HEMPTY || old == key64) break;
-          slot = (slot + 1) & (HS - 1);
+      ql[rr] = false;
+      if (rr * WAVE >= tail) continue;
+      ql[rr] = khi[rr] < sigma || (khi[rr] == mh && klo[rr] == f1);
+      const uint64_t qb = __builtin_amdgcn_ballot_w64(ql[rr]);
+      if (qb) {
+        const int pos = nl + lanes_below(qb);
+        if (ql[rr]) {
+          const int s = rr * WAVE + lane;
+          if (pos < BMAX) cs[pos] = s;
+          flo[s] = klo[rr];
+          flogw[s] = klw[rr];
         }
-        hid[slot] = id;
+        nl += __builtin_popcountll(qb);
       }
     }
-    hashed = count;
-    // candidates: heads below sigma (f1 in any case) and their siblings while below sigma and not below
-    // their elder, at most WALK per list; walked in registers (a frontier with LDS rows is not batched)
-    uint32_t hk[RR][WALK];
-    double wv[RR][WALK];
-    int nc[RR];
-    bool too_long = false;
-    {
-      float lpv[RR][WALK + 1];
-      float prr[RR];
+    if (nl > BMAX) return false;
+    wave_sync();
+    int nb;
+    if (nl <= FEW) {
+      // few lists: 64 / nl lanes each, lane t of list li the list's t-th sibling from its head on; logw by the heap's
+      // own chain of roundings
+      const int lw = BMAX / nl;
+      const int li = lane / lw, lt = lane - li * lw;
+      const bool in = li < nl;
+      const int lslot = cs[in ? li : 0];
+      const uint32_t lf = flo[lslot];
+      const int lm = (int)(lf >> 28), lr0 = (int)(lf & 0x3FF);
+      const int2* lrec = rec + (lm * L + (int)((lf >> 10) & 0x3F) - 1) * kk + lr0;
+      const int left = kk - 1 - lr0;  // siblings after the head
+      const float lpr = sprior[lm];
+      double cw = flogw[lslot];
+      float clp = __int_as_float(lrec[0].y);
+      const int tmax = min(lw - 1, kk - 1);
+      for (int i0 = 0; i0 < tmax; i0 += 8) {
+        float nx[8];
 #pragma unroll
-      for (int rr = 0; rr < RR; ++rr) {
-        const bool q = khi[rr] != NONE && (khi[rr] < sigma || (khi[rr] == mh && klo[rr] == f1));
-        nc[rr] = q ? 1 : 0;
-        const uint32_t fl0 = q ? klo[rr] : 0u;
-        const int m = (int)(fl0 >> 28), row = q ? (int)((fl0 >> 10) & 0x3F) - 1 : 0;
-        const int r0 = (int)(fl0 & 0x3FF);
+        for (int u = 0; u < 8; ++u) nx[u] = __int_as_float(lrec[min(i0 + u + 1, left)].y);
 #pragma unroll
-        for (int t = 0; t <= WALK; ++t) lpv[rr][t] = lp_at(m, row, min(r0 + t, kk - 1));
-        prr[rr] = sprior[m];
+        for (int u = 0; u < 8; ++u) {
+          const double wn = (cw - (double)clp) + (double)nx[u];
+          const bool go = i0 + u < lt;
+          cw = go ? wn : cw;
+          clp = go ? nx[u] : clp;
+        }
       }
+      const uint32_t ckey = key_bits(-((float)cw + lpr));
+      // the first sibling no lane forms bounds the batch
+      uint32_t bound = NONE;
+      if (in && lt == lw - 1 && lt < left)
+        bound = key_bits(-((float)((cw - (double)clp) + (double)__int_as_float(lrec[lt + 1].y)) + lpr));
+      const uint32_t sig2 = umin32(sigma, wave_min_u32(bound));
+      // a list ends before a sibling whose key lies below its elder's
+      const uint32_t pkey = (uint32_t)__builtin_amdgcn_ds_bpermute((lane - 1) << 2, (int)ckey);
+      const uint64_t bad = __builtin_amdgcn_ballot_w64(in && lt > 0 && lt <= left && ckey < pkey);
+      const uint64_t upto = (~0ull >> (63 - lane)) & (~0ull << (lane - lt));
+      const bool take = in && lt <= left && (bad & upto) == 0 && (ckey < sig2 || (lt == 0 && ckey == mh && lf == f1));
+      const uint64_t tb = __builtin_amdgcn_ballot_w64(take);
+      nb = __builtin_popcountll(tb);
+      if (nb < BMIN) return false;
+      wave_sync();
+      if (take) {
+        const int pos = lanes_below(tb);
+        c64[pos] = ((uint64_t)ckey << 32) | (lf + (uint32_t)lt);
+        clw[pos] = cw;
+        cs[pos] = lslot;
+      }
+    } else {
+      // many lists: a lane each, up to WALK entries of it; sigma lowered until at most 64 entries lie below
+      constexpr int WALK = 6;
+      const bool in = lane < nl;
+      const int lslot = cs[in ? lane : 0];
+      const uint32_t lf = flo[lslot];
+      const int lm = (int)(lf >> 28), lr0 = (int)(lf & 0x3FF);
+      const int2* lrec = rec + (lm * L + (int)((lf >> 10) & 0x3F) - 1) * kk + lr0;
+      const int left = kk - 1 - lr0;
+      const float lpr = sprior[lm];
+      float nx[WALK + 1];
 #pragma unroll
-      for (int rr = 0; rr < RR; ++rr) {
-        const int r0 = (int)(klo[rr] & 0x3FF);
-        hk[rr][0] = khi[rr];
-        wv[rr][0] = klw[rr];
+      for (int t = 0; t <= WALK; ++t) nx[t] = __int_as_float(lrec[min(t, left)].y);
+      double wv[WALK + 1];
+      uint32_t hk[WALK + 1];  // NONE from the list's end, and from a sibling whose key lies below its elder's
+      wv[0] = flogw[lslot];
+      hk[0] = in ? key_bits(-((float)wv[0] + lpr)) : NONE;
 #pragma unroll
-        for (int t = 1; t <= WALK; ++t) {
-          if (nc[rr] == t && r0 + t < kk) {
-            const double wn = (wv[rr][t - 1] - (double)lpv[rr][t - 1]) + (double)lpv[rr][t];
-            const uint32_t hn = key_bits(-((float)wn + prr[rr]));
-            if (hn < sigma && hn >= hk[rr][t - 1]) {
-              if (t < WALK) {
-                hk[rr][t] = hn;
-                wv[rr][t] = wn;
-                nc[rr] = t + 1;
-              } else {
-                too_long = true;
-              }
-            }
+      for (int t = 1; t <= WALK; ++t) {
+        wv[t] = (wv[t - 1] - (double)nx[t - 1]) + (double)nx[t];
+        const uint32_t h = key_bits(-((float)wv[t] + lpr));
+        hk[t] = (hk[t - 1] != NONE && t <= left && h >= hk[t - 1]) ? h : NONE;
+      }
+      uint32_t sig2 = umin32(sigma, wave_min_u32(hk[WALK]));
+      auto below = [&](uint32_t key) -> int {
+        int n = 0;
+#pragma unroll
+        for (int t = 0; t < WALK; ++t) n += __builtin_popcountll(__builtin_amdgcn_ballot_w64(hk[t] < key));
+        return n;
+      };
+      int nbelow = below(sig2);
+      if (nbelow > BMAX) {
+        uint32_t lo = mh, hi = sig2;
+        nbelow = 0;
+        for (int it = 0; it < 16; ++it) {
+          const uint32_t mid = lo + (hi - lo) / 2;
+          const int n = below(mid);
+          if (n > BMAX) {
+            hi = mid;
+          } else {
+            lo = mid;
+            nbelow = n;
+            if (n > BMAX - 16) break;
           }
         }
+        sig2 = lo;
       }
-    }
-    // positions: exclusive prefix of the per-lane counts over the lanes (bit by bit through ballots)
-    int c_lane = 0;
+      if (nbelow < BMIN) return false;
+      wave_sync();
+      int c = 0;
 #pragma unroll
-    for (int rr = 0; rr < RR; ++rr) c_lane += nc[rr];
-    const uint64_t below_l = lane == 0 ? 0ull : (~0ull >> (64 - lane));
-    int base = 0, nb = 0;
+      for (int t = 0; t < WALK; ++t) c += hk[t] < sig2 ? 1 : 0;
+      int base = 0;
+      nb = 0;
 #pragma unroll
-    for (int bit = 0; bit < 5; ++bit) {
-      const uint64_t bb = __builtin_amdgcn_ballot_w64((c_lane >> bit) & 1);
-      base += __builtin_popcountll(bb & below_l) << bit;
-      nb += __builtin_popcountll(bb) << bit;
-    }
-    if (nb > BMAX || __builtin_amdgcn_ballot_w64(too_long) != 0) return false;
-#pragma unroll
-    for (int rr = 0; rr < RR; ++rr) {
-      const int s = rr * WAVE + lane;
+      for (int bit = 0; bit < 3; ++bit) {  // exclusive prefix of the counts, bit by bit through ballots
+        const uint64_t bb = __builtin_amdgcn_ballot_w64((c >> bit) & 1);
+        base += lanes_below(bb) << bit;
+        nb += __builtin_popcountll(bb) << bit;
+      }
 #pragma unroll
       for (int t = 0; t < WALK; ++t)
-        if (t < nc[rr]) {
-          ck[base + t] = hk[rr][t];
-          cf[base + t] = (klo[rr] & ~0x3FFu) | (uint32_t)((klo[rr] & 0x3FF) + t);
-          clw[base + t] = wv[rr][t];
-          cs[base + t] = s;
+        if (t < c) {
+          c64[base + t] = ((uint64_t)hk[t] << 32) | (lf + (uint32_t)t);
+          clw[base + t] = wv[t];
+          cs[base + t] = lslot;
         }
-      base += nc[rr];
     }
-    __syncthreads();
-    uint32_t ekey = NONE, efld = NONE;
+    // (NONE, NONE) up to a multiple of four orders after every candidate
+    if (lane >= nb && lane < ((nb + 3) & ~3)) c64[lane] = ~0ull;
+    // the nodes made by sequential pops since the last batch into the hash table
+    if (hashed < count) {
+#pragma unroll
+      for (int r = 0; r < NR; ++r) {
+        const int id = 64 * r + lane + 1;
+        if (id > hashed && id <= count) {
+          const uint64_t key64 = ((uint64_t)(uint32_t)rpar[r] << 32) | (uint32_t)rtok[r];
+          int slot = (int)(hash_pt(rpar[r], rtok[r]) & (uint32_t)(HS - 1));
+          for (int probe = 0; probe < HS; ++probe) {
+            const uint64_t old = atomicCAS(reinterpret_cast<unsigned long long*>(&hkey[slot]),
+                                           (unsigned long long)HEMPTY, (unsigned long long)key64);
+            if (old == HEMPTY || old == key64) break;
+            slot = (slot + 1) & (HS - 1);
+          }
+          hid[slot] = id;
+        }
+      }
+      hashed = count;
+    }
+    wave_sync();
+    uint64_t e64 = ~0ull;
     double ew = 0.0;
-    int eslot = 0;
+    int eslot = 0, enext = BMAX;
     if (lane < nb) {
-      ekey = ck[lane];
-      efld = cf[lane];
+      e64 = c64[lane];
       ew = clw[lane];
       eslot = cs[lane];
     }
-    // order: lane i takes the candidate of rank i. Every lane compares its candidate with all of them, read
-    // four at a time (the same LDS words for every lane: broadcast reads); the tail up to a multiple of four
-    // holds (NONE, NONE), which orders after every candidate.
-    const int nb4 = (nb + 3) & ~3;
-    if (lane >= nb && lane < nb4) {
-      ck[lane] = NONE;
-      cf[lane] = NONE;
-    }
-    __syncthreads();
-    // (key, fields) as one 64-bit word; equal words (only with repeated ids in a top list) rank by lane
-    const uint64_t me64 = ((uint64_t)ekey << 32) | efld;
+    // order: lane i takes the candidate of rank i. Every lane compares its candidate with all of them, read two at a
+    // time (the same LDS words for every lane: broadcast reads), as one 64-bit word (key, fields)
     int rank_o = 0;
-    for (int j = 0; j < nb4; j += 4) {
-      const uint4 k4 = *reinterpret_cast<const uint4*>(ck + j);
-      const uint4 f4 = *reinterpret_cast<const uint4*>(cf + j);
-      const uint64_t c0 = ((uint64_t)k4.x << 32) | f4.x, c1 = ((uint64_t)k4.y << 32) | f4.y;
-      const uint64_t c2 = ((uint64_t)k4.z << 32) | f4.z, c3 = ((uint64_t)k4.w << 32) | f4.w;
-      rank_o += (int)(c0 < me64) + (int)(c1 < me64) + (int)(c2 < me64) + (int)(c3 < me64);
-      rank_o += (int)(c0 == me64 && j < lane) + (int)(c1 == me64 && j + 1 < lane) + (int)(c2 == me64 && j + 2 < lane) +
-                (int)(c3 == me64 && j + 3 < lane);
+    typedef uint64_t u64x2 __attribute__((ext_vector_type(2)));
+    for (int j = 0; j < nb; j += 4) {
+      const u64x2 x = *reinterpret_cast<const u64x2*>(c64 + j), y = *reinterpret_cast<const u64x2*>(c64 + j + 2);
+      rank_o += (int)(x[0] < e64) + (int)(x[1] < e64) + (int)(y[0] < e64) + (int)(y[1] < e64);
     }
-    __syncthreads();
-    if (lane < nb) {
-      ck[rank_o] = ekey;
-      cf[rank_o] = efld;
-      clw[rank_o] = ew;
-      cs[rank_o] = eslot;
+    // equal words (only with repeated ids in a top list) share a rank; then they rank by lane
+    wave_sync();
+    if (lane < nb) cs[rank_o] = lane;
+    wave_sync();
+    if (__builtin_amdgcn_ballot_w64(lane < nb && cs[rank_o] != lane) != 0)
+      for (int j = 0; j < nb; ++j) rank_o += (int)(c64[j] == e64 && j < lane);
+    wave_sync();
+    // a list's entries are consecutive candidates: the place of an entry's next sibling in the order (64: not among them)
+    {
+      const int nplace = __builtin_amdgcn_ds_bpermute((lane + 1) << 2, rank_o);
+      const int nslot = __builtin_amdgcn_ds_bpermute((lane + 1) << 2, lane < nb ? eslot : -1);
+      if (lane < nb) {
+        c64[rank_o] = e64;
+        clw[rank_o] = ew;
+        cs[rank_o] = eslot | ((lane + 1 < nb && nslot == eslot ? nplace : BMAX) << 16);
+      }
     }
-    __syncthreads();
+    wave_sync();
     const bool cand = lane < nb;
     if (cand) {
-      ekey = ck[lane];
-      efld = cf[lane];
+      e64 = c64[lane];
       ew = clw[lane];
-      eslot = cs[lane];
+      eslot = cs[lane] & 0xFFFF;
+      enext = cs[lane] >> 16;
     }
+    const uint32_t efld = (uint32_t)e64;
     const int m = cand ? (int)(efld >> 28) : 0;
     const int parent = (int)((efld >> 16) & 0xFFF);
     const int depth = cand ? (int)((efld >> 10) & 0x3F) : 1;
@@ -474,15 +578,10 @@ __global__ __launch_bounds__(WAVE) void build_mixture_kernel(BuildArgs a) {
       nfld = (efld & ~0x3FFu) | (uint32_t)(rank + 1);
     }
     // cut after an entry whose list's next sibling orders before the next batch entry
-    if (cand) atomicMax(&fmax[eslot], rank);
-    __syncthreads();
-    const bool last_of_list = cand && fmax[eslot] == rank;
-    const uint32_t kn = lane + 1 < nb ? ck[lane + 1] : NONE;
-    const uint32_t fn = lane + 1 < nb ? cf[lane + 1] : NONE;
-    __syncthreads();
-    if (last_of_list) fmax[eslot] = -1;
+    const bool last_of_list = cand && enext == BMAX;
+    const uint64_t next64 = lane + 1 < nb ? c64[lane + 1] : ~0ull;
     const uint64_t cuts =
-        __builtin_amdgcn_ballot_w64(last_of_list && lane + 1 < nb && has_next && pair_lt(nkey, nfld, kn, fn));
+        __builtin_amdgcn_ballot_w64(last_of_list && lane + 1 < nb && has_next && (((uint64_t)nkey << 32) | nfld) < next64);
     if (cuts != 0) nb = (int)__builtin_ctzll(cuts) + 1;
     // nodes: (parent, token) in the hash table; the first lane of a new prefix creates it, ids in batch order,
     // and the batch ends with the pop that creates node number budget
@@ -507,7 +606,7 @@ __global__ __launch_bounds__(WAVE) void build_mixture_kernel(BuildArgs a) {
       if (!existing) atomicMin(&hmin[slot], lane);
     }
     if (__builtin_amdgcn_ballot_w64(lost) != 0) overflow = true;  // kept wave-uniform
-    __syncthreads();
+    wave_sync();
     const bool creator = contend && !existing && hmin[slot] == lane;
     const uint64_t cre = __builtin_amdgcn_ballot_w64(creator);
     const int need = budget - count;
@@ -527,7 +626,7 @@ __global__ __launch_bounds__(WAVE) void build_mixture_kernel(BuildArgs a) {
     }
     // a creator cut off above releases the slot for later steps (the key stays, without a node)
     if (creator && !live) hmin[slot] = 0x7FFFFFFF;
-    __syncthreads();
+    wave_sync();
     const int enode = live ? (creator ? id : hid[slot]) : 0;
     const int count_new = count + __builtin_popcountll(cre & (nb >= 64 ? ~0ull : ((1ull << nb) - 1)));
 #pragma unroll
@@ -543,12 +642,9 @@ __global__ __launch_bounds__(WAVE) void build_mixture_kernel(BuildArgs a) {
     hashed = count;
     // each list moves its head past its last popped entry; popped entries below depth L open their children's
     // lists in new slots
-    if (live) atomicMax(&fmax[eslot], rank);
-    __syncthreads();
-    const bool last = live && fmax[eslot] == rank;
-    __syncthreads();
+    const bool last = live && enext >= nb;
     if (last) {
-      fmax[eslot] = -1;
+      fmax[eslot] = -2;  // moved
       if (has_next) {
         fhi[eslot] = nkey;
         flo[eslot] = nfld;
@@ -563,7 +659,7 @@ __global__ __launch_bounds__(WAVE) void build_mixture_kernel(BuildArgs a) {
     alive -= __builtin_popcountll(__builtin_amdgcn_ballot_w64(last && !has_next));
     const bool opens = live && depth < L;
     const uint64_t op = __builtin_amdgcn_ballot_w64(opens);
-    const int nnew = __builtin_popcountll(op);
+    const int nnew = __builtin_popcountll(op), told = tail;
     if (tail + nnew > cap) {
       overflow = true;
       return true;
@@ -578,20 +674,23 @@ __global__ __launch_bounds__(WAVE) void build_mixture_kernel(BuildArgs a) {
     }
     tail += nnew;
     alive += nnew;
-    __syncthreads();
-    // LDS rows back to the registers, then every lane's best and prefetch
+    wave_sync();
+    // the moved heads and the new slots back to the registers, then every lane's best and prefetch
 #pragma unroll
     for (int rr = 0; rr < RR; ++rr) {
+      if (rr * WAVE >= tail) continue;
       const int s = rr * WAVE + lane;
-      const bool in = s < tail;
-      khi[rr] = in ? fhi[s] : NONE;
-      klo[rr] = in ? flo[s] : NONE;
-      kck[rr] = in ? fck[s] : NONE;
-      klw[rr] = in ? flogw[s] : 0.0;
+      if ((ql[rr] && fmax[s] == -2) || (s >= told && s < tail)) {
+        khi[rr] = fhi[s];
+        klo[rr] = flo[s];
+        kck[rr] = fck[s];
+        klw[rr] = flogw[s];
+      }
+      if (ql[rr]) fmax[s] = -1;
     }
     rescan(tail);
     prefetch();
-    __syncthreads();
+    wave_sync();
     return true;
   };
   // every iteration pops at least one frontier entry and at most cap entries are ever pushed: bounded loop
@@ -605,18 +704,13 @@ __global__ __launch_bounds__(WAVE) void build_mixture_kernel(BuildArgs a) {
       win = (int)__builtin_ctzll(__builtin_amdgcn_ballot_w64(lhi == mh && llo == ml));
     }
     const uint32_t f = __builtin_amdgcn_readlane(llo, win);
-    // ---- batch step when enough heads lie below sigma. Checked 4 steps after a batch, then at gaps that
-    //      double (up to 32) while the checks find none.
+    // ---- batch step. Tried again right after one that was taken, then at gaps that double (up to 32) while it finds
+    //      too little.
     bool batched = false;
     if (iter == next_check && HS > 0) {
-      const uint32_t sigma = wave_min_u32(lcm);
-      int nheads = 0;
-#pragma unroll
-      for (int rr = 0; rr < RR; ++rr)
-        nheads += __builtin_popcountll(__builtin_amdgcn_ballot_w64(khi[rr] < sigma));
-      if (nheads >= BMIN) batched = batch_step(f, mh, sigma);
+      batched = batch_step(f, mh, wave_min_u32(lcm));
       if (overflow) break;
-      gap = batched ? 4 : min(2 * gap, 32);
+      gap = batched ? 1 : min(2 * gap, 32);
       next_check = iter + gap;
     }
     if (batched) continue;
@@ -736,9 +830,9 @@ __global__ __launch_bounds__(WAVE) void build_mixture_kernel(BuildArgs a) {
       ndep[j + 1] = rdep[r];
     }
   }
-  __builtin_amdgcn_s_waitcnt(0);
+  if (lane == 0) scnt[0] = count;
   __syncthreads();
-  write_tree(a, b, lane, count, npar, ntok, ndep);
+  write_tree(a, b, (int)threadIdx.x, MNT, count, npar, ntok, ndep);
 }
 
 // ---- single-mode DDTree heap (inference/hf/tree_build_ext.py:31-46 SingleEntry / SingleGreater, :118-156
@@ -930,9 +1024,11 @@ __global__ __launch_bounds__(WAVE) void build_single_kernel(BuildArgs a) {
     }
   }
   if (overflow && lane == 0 && a.err) atomicOr(a.err, 1);
+  if (a.anc8) zero_anc8(a, b, lane, WAVE);
   __builtin_amdgcn_s_waitcnt(0);
+  __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
   __builtin_amdgcn_wave_barrier();
-  write_tree(a, b, lane, count, npar, ntok, ndep);
+  write_tree(a, b, lane, WAVE, count, npar, ntok, ndep);
 }
 
 }  // namespace
@@ -967,7 +1063,7 @@ template <int NR>
 int launch_build(const BuildArgs& a, int smem, hipStream_t st) {
   const int rc = mfd_set_max_lds(reinterpret_cast<const void*>(&build_mixture_kernel<NR>), 160 * 1024);
   if (rc != MFD_OK) return rc;
-  hipLaunchKernelGGL(build_mixture_kernel<NR>, dim3(a.bs), dim3(WAVE), smem, st, a);
+  hipLaunchKernelGGL(build_mixture_kernel<NR>, dim3(a.bs), dim3(MNT), smem, st, a);
   MFD_CHECK_LAUNCH();
   return MFD_OK;
 }

@@ -235,6 +235,36 @@ def test_hf_build_mixture_contract_and_follow():
     assert accepted == path and bonus == 7
 
 
+@pytest.mark.parametrize("K,L,k,budget,kind", [
+    (1, 16, 256, 256, "flat"),   # one list shared by all lanes, then more than 64 lists
+    (4, 8, 256, 256, "flat"), (8, 15, 8, 256, "flat"), (4, 9, 128, 128, "flat"), (8, 16, 64, 64, "flat"),
+    (3, 7, 100, 200, "ties"), (6, 4, 33, 129, "ties"), (7, 12, 20, 65, "peaky"), (2, 3, 5, 100, "ties"),
+    (8, 6, 16, 300, "shared"),   # every mode pops the same prefixes: more pops than register slots
+])
+def test_batches_of_many_and_long_lists(K, L, k, budget, kind):
+    """The batch step's two forms (lanes shared by a few lists, one lane per list) and the sequential pops between
+    them, against the sequential heap: flat log-probs pop long runs of siblings, peaky ones deep prefixes."""
+    import tree_build_ext
+
+    g = torch.Generator().manual_seed(K * 1000 + L * 100 + k)
+    scale = {"flat": 1.0, "ties": 1.0, "peaky": 6.0, "shared": 1.0}[kind]
+    x = torch.randn(K, L, 4 * k + 8, generator=g) * scale
+    if kind == "shared":
+        x = x[:1].expand(K, -1, -1) + torch.randn(K, 1, 1, generator=g) * 1e-3
+    lp, ids = torch.topk(torch.log_softmax(x, -1), k, dim=-1)
+    if kind == "ties":
+        lp = (lp * 4).round() / 4
+    prior = torch.log_softmax(torch.randn(K, generator=g), 0)
+    print(f"case: batches K={K} L={L} k={k} budget={budget} {kind}", flush=True)
+    tree, counts, anc8 = tree_build_ext.build_trees_device(lp[None].cuda(), ids[None].to(torch.int32).cuda(),
+                                                           prior[None].cuda(), budget, with_visibility=True)
+    torch.cuda.synchronize()
+    t, d, p, n, _ = B.build_mixture(lp.numpy(), ids.numpy(), prior.numpy(), budget)
+    assert int(counts[0]) == n
+    np.testing.assert_array_equal(tree[0].cpu().numpy(), np.stack([t, d, p]))
+    np.testing.assert_array_equal(anc8[0, : n + 1, : n + 1].cpu().numpy().astype(bool), B.visibility(p, n).astype(bool))
+
+
 def test_budget_zero_and_exhausted_heap():
     import tree_build_ext
 
