@@ -90,6 +90,24 @@ def test_paged_per_token_table(lens, splits):
     _check(got, _paged_ref(d), f"paged1 {lens}")
 
 
+@pytest.mark.parametrize("lens,H,Hkv,K,splits,page_size", [
+    ([0, 5, 3000, 64, 129], 16, 8, 8, -1, 64),           # split, whole and empty requests side by side
+    ([700] + [30] * 70, 8, 2, 2, -1, 1),                 # more than 64 requests, one of them split
+    ([3000] + list(range(1, 71)), 8, 8, 2, 5, 64),       # more workgroups than the chip holds: longest first
+    ([0, 0, 0], 8, 4, 3, 4, 1), ([128, 129, 127], 8, 4, 8, 16, 64), ([4097, 1], 32, 4, 1, -1, 16),
+])
+def test_paged_split_batches(lens, H, Hkv, K, splits, page_size):
+    """Batches whose requests take as many splits as their lengths ask for: every split count from one (which writes
+    the output itself) to the limit, no request left out and none read past its end."""
+    d = paged_attention_inputs(90 + len(lens), lens, K=K, H=H, Hkv=Hkv, page_size=page_size)
+    table = torch.zeros(len(lens) + 2, d["page_table"].shape[1], dtype=torch.int32)
+    table[2:] = d["page_table"]
+    print(f"case: split batch lens={lens[:6]} bs={len(lens)} H={H}/{Hkv} K={K} splits={splits}", flush=True)
+    got = _paged(d, page_size, splits, d["req_to_token"] if page_size == 1 else table)
+    torch.cuda.synchronize()
+    _check(got, _paged_ref(d), f"split batch {lens[:6]}")
+
+
 def test_paged_64_token_pages_config4_heads():
     """Config 4 attention shapes (40 q heads over 8 KV heads, K=8 x 16), 64-token pages, U[1024, 8192] contexts."""
     g = torch.Generator().manual_seed(4000)
