@@ -3,7 +3,10 @@
 // single entry point (the product, then the logits step of logits_topk.hip on its output).
 //
 // The product streams the weight (vocabulary x hidden, bf16, read once per 128 drafted rows: 778 MB at a
-// 151936-token vocabulary and hidden 2560) against the drafted rows, which every workgroup shares.
+// 151936-token vocabulary and hidden 2560) against the drafted rows, which every workgroup shares. Three forms, by
+// the drafted rows and the vocabulary rows a CU gets (draft_head_gemm): the k-split form (few drafted rows, or a vocabulary so
+// small that one wave's walk over k would be the whole time), the wide form (more than 128 rows per CU) and, between
+// them, the pass form described here.
 //  * The vocabulary is split evenly over the grid's workgroups (one per CU; ranges of a multiple of 8 rows),
 //    each taking its range in passes of 128 weight rows against all (up to 128) drafted rows.
 //  * Both operands stream through LDS in 64-k stages (128 weight rows and 128 drafted rows, 128 bytes each,
@@ -279,34 +282,61 @@ __global__ __launch_bounds__(NT) void draft_head_kernel(HeadArgs a) {
 }
 
 
-// ---- Wide form, for workgroup ranges of more than one 128-row pass (the full vocabulary). The pass form reads
-//      all drafted rows again for every pass, so at 600 weight rows per workgroup the per-CU load path carries
-//      the drafted rows 4.7 times next to the weight; here every workgroup holds accumulators for its whole
-//      range (up to WRMAX rows) and streams k once, so the drafted rows pass through it once.
-//  * Eight waves (two per SIMD); wave w owns weight rows 80 w .. 80 w + 79 of the range (5 tiles of 16) against
-//    all 128 drafted rows (8 tiles): 40 v_mfma_f32_16x16x32_bf16 accumulators (160 registers).
-//  * Stages of 32 k (one MFMA depth): the range's weight rows and the drafted rows, 64 bytes each (48 KB), in a
-//    ring of three; every wave issues its own direct-to-LDS loads (its 80 weight rows and 16 drafted rows: six
-//    1-KB loads per stage), stage v + 2 going out once the barrier of stage v has freed its slot.
-//  * 16-byte chunk c of staged row r sits at position c ^ ((r >> 2) & 3), so the 16 rows of a fragment read hit
-//    distinct banks; a load's lane l fills row l / 4 of its 16 rows at position l % 4.
+// C registers of a tile pair to bf16 and out: weight rows n .. n + 3 of the range, drafted row's output at orow.
+__device__ __forceinline__ void store4(uint16_t* orow, int n, int rows, const f32x4& c) {
+  const u32x2 pk = {__builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2){c[0], c[1]}, bf16x2)),
+                    __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2){c[2], c[3]}, bf16x2))};
+  if (n + 4 <= rows) {
+    *reinterpret_cast<u32x2*>(orow + n) = pk;
+  } else {
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      if (n + e < rows) orow[n + e] = (uint16_t)(pk[e >> 1] >> (16 * (e & 1)));
+  }
+}
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_of(const uint16_t* base, uint32_t bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(base), (short)0, (int)bytes, 0x00020000);
+}
+__device__ __forceinline__ bf16x8 buffer_load8(__amdgpu_buffer_rsrc_t rs, uint32_t off, uint32_t soff) {
+  return __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(rs, off, soff, 0));
+}
+// Byte offset of the launch's drafted row r (rows past the last repeat it).
+__device__ __forceinline__ uint32_t drafted_off(const HeadArgs& a, int r) {
+  const int m = a.row0 + min(r, a.M - 1);
+  return (uint32_t)(((int64_t)(m / a.rpg) * a.group_stride + (int64_t)(m % a.rpg) * a.row_stride) * 2);
+}
+
+// ---- Wide form, for workgroup ranges of more than one 128-row pass. The pass form reads all drafted rows again for
+//      every pass; here a workgroup holds accumulators for its whole range (up to WRMAX rows) and walks k once.
+//      Bound by the weight's way from memory.
+//  * Eight waves (two per SIMD) share the range's 16-row tiles evenly, each up to VTW neighbouring ones against all
+//    128 drafted rows (8 tiles): 8 VTW v_mfma_f32_16x16x32_bf16 accumulators (160 registers at VTW 5). VTW follows
+//    the range, so that a short one does not carry the registers and the code of a long one.
+//  * The weight goes straight to registers, 64 k (128 bytes of a row) at a time: a fragment takes 64 bytes of each of
+//    its 16 rows, and both halves of the row's 128-byte line are loaded back to back, after the products that last
+//    read the registers. (Stages of 32 k through LDS fetched every line from L2 twice, the second half long after the
+//    first had left the CU's cache: 182 us at 151936 x 2560 x 120, 4.27 TB/s; so 163 us, 4.77 TB/s.)
+//    Rows past the range read as zero by the buffer's bound.
+//  * The drafted rows are in LDS as blocks of 256 k (512 bytes a row, 64 KB), double buffered by direct-to-LDS loads,
+//    one barrier per block; 16-byte chunk c of row r sits at c ^ (r & 15), so the 16 rows of a fragment read hit
+//    distinct banks.
 namespace wide {
 constexpr int NW = 8;
 constexpr int NTH = NW * 64;
-constexpr int VTW = 5;                   // 16-row weight tiles per wave
-constexpr int WRMAX = NW * VTW * 16;     // weight rows per workgroup (640)
+constexpr int WRMAX = NW * 5 * 16;       // weight rows per workgroup (640)
 constexpr int MTL = MT / 16;             // drafted-row tiles (8)
-constexpr int KSW = 32;                  // k per stage
-constexpr int RB = KSW * 2;              // bytes of a staged row (64)
-constexpr int WBW = WRMAX * RB;          // weight block (40 KB)
-constexpr int SBW = WBW + MT * RB;       // a stage (48 KB)
-constexpr int NBW = 3;                   // ring depth (144 KB)
-constexpr int SMEMW = NBW * SBW;
-constexpr int LPW = VTW + 1;             // 1-KB loads per wave and stage: VTW weight, 1 drafted
+constexpr int KSW = 32;                  // k per step
+constexpr int HS = 8;                    // steps per drafted block
+constexpr int HRB = HS * KSW * 2;        // bytes of a drafted row's block (512)
+constexpr int HBW = MT * HRB;            // drafted block (64 KB)
+constexpr int SMEMW = 2 * HBW;
 }  // namespace wide
 
-__global__ __launch_bounds__(wide::NTH) __attribute__((amdgpu_waves_per_eu(2, 2))) void draft_head_wide_kernel(HeadArgs a) {
+template <int VTW>
+__global__ __launch_bounds__(wide::NTH) __attribute__((amdgpu_waves_per_eu(2, 2))) void draft_head_wide_kernel(
+    HeadArgs a) {
   using namespace wide;
+  static_assert(VTW >= 2 && VTW <= 5, "tiles of a wave");
   extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
   const int tid = threadIdx.x, lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -314,94 +344,195 @@ __global__ __launch_bounds__(wide::NTH) __attribute__((amdgpu_waves_per_eu(2, 2)
   const int rows = wg_row0(blockIdx.x + 1, a.N, a.nwg) - R0;
   if (rows <= 0) return;
   const int K = a.K;
-  const int S = K / KSW;
-  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)smem;
-  // load side: lane l fills row (16-row group base) + l / 4 at position l % 4, so it reads chunk
-  // (l % 4) ^ ((l / 16) % 4) of that row (the group base is a multiple of 16)
-  const int lrow = lane >> 2;
-  const int lchunk = (lane & 3) ^ ((lane >> 4) & 3);
-  const uint16_t* wbase = a.w + (int64_t)R0 * K;
-  uint32_t hoff;
-  {
-    const int m = a.row0 + min(16 * w + lrow, a.M - 1);
-    hoff = (uint32_t)(((int64_t)(m / a.rpg) * a.group_stride + (int64_t)(m % a.rpg) * a.row_stride + 8 * lchunk) * 2);
-  }
-  // weight tiles of this wave that hold rows of the range (tiles wholly past it are neither loaded nor computed)
-  const int vtv = __builtin_amdgcn_readfirstlane(max(0, min(VTW, (rows - VTW * 16 * w + 15) / 16)));
-  auto issue = [&](int v) __attribute__((always_inline)) {
-    const uint32_t slot = lds0 + (uint32_t)(v % NBW) * SBW;
-    const uint32_t kb = (uint32_t)v * RB;
-#pragma unroll
-    for (int i = 0; i < VTW; ++i) {
-      if (i >= vtv) break;
-      // tile i of the wave: rows 80 w + 16 i .. ; rows past the range repeat the last one
-      const int r = min(VTW * 16 * w + 16 * i + lrow, rows - 1);
-      const uint32_t off = (uint32_t)r * (uint32_t)(2 * K) + (uint32_t)(16 * lchunk) + kb;
-      dma16(wbase, off, slot + (uint32_t)(VTW * 16 * w + 16 * i) * RB);
-    }
-    dma16(a.hidden, hoff + kb, slot + WBW + (uint32_t)(16 * w) * RB);
-  };
-
-  // read side: fragment of row (tile base) + l16, chunk g4 at position g4 ^ ((l16 >> 2) & 3)
+  const int S = K / KSW;  // even
   const int l16 = lane & 15, g4 = lane >> 4;
-  const uint32_t fro = (uint32_t)(l16 * RB + ((g4 ^ ((l16 >> 2) & 3)) << 4));
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)smem;
+  // drafted block b (k 256 b ..): a load moves two rows of 512 bytes (past the last k: its last chunk, never read)
+  auto issue_h = [&](int b) __attribute__((always_inline)) {
+    const uint32_t slot = lds0 + (uint32_t)(b & 1) * HBW;
+#pragma unroll
+    for (int i = 0; i < MT / 2 / NW; ++i) {
+      const int r = 2 * (i * NW + w) + (lane >> 5);
+      const int c = (lane & 31) ^ (r & 15);
+      const int kc = min(b * (HS * KSW) + 8 * c, K - 8);
+      dma16(a.hidden, drafted_off(a, r) + 2u * (uint32_t)kc, slot + (uint32_t)(2 * (i * NW + w)) * HRB);
+    }
+  };
+  // this wave's tiles t0 .. t0 + vtv - 1 of the range's
+  const int T = (rows + 15) / 16;
+  const int t0 = __builtin_amdgcn_readfirstlane(w * T / NW);
+  const int vtv = __builtin_amdgcn_readfirstlane((w + 1) * T / NW) - t0;
+  const __amdgpu_buffer_rsrc_t rs = buffer_of(a.w + (int64_t)R0 * K, (uint32_t)rows * (uint32_t)K * 2u);
+  const uint32_t woff = ((uint32_t)(16 * t0 + l16) * (uint32_t)K + 8u * g4) * 2u;
+  const uint32_t tstep = 32u * (uint32_t)K;  // bytes from a tile to the next
   f32x4 acc[VTW][MTL];
 #pragma unroll
   for (int i = 0; i < VTW; ++i)
 #pragma unroll
     for (int j = 0; j < MTL; ++j) acc[i][j] = (f32x4){};
-
-  issue(0);
-  if (S > 1) issue(1);
-  for (int v = 0; v < S; ++v) {
-    // this wave's loads of stage v have landed (stage v + 1's vtv + 1 may not)
-    if (v + 1 < S) {
-      switch (vtv) {
-        case 0: wait_vmcnt<1>(); break;
-        case 1: wait_vmcnt<2>(); break;
-        case 2: wait_vmcnt<3>(); break;
-        case 3: wait_vmcnt<4>(); break;
-        case 4: wait_vmcnt<5>(); break;
-        default: wait_vmcnt<LPW>(); break;
-      }
-    } else {
+  bf16x8 wf[2][VTW];
+  // (i < vtv: the tile and step offset stays below the buffer's size, which the bounds check needs)
+  auto load_w = [&](int v, int i) __attribute__((always_inline)) -> bf16x8 {
+    return buffer_load8(rs, woff, (uint32_t)i * tstep + (uint32_t)(min(v, S - 1) * (KSW * 2)));
+  };
+  issue_h(0);
+#pragma unroll
+  for (int i = 0; i < VTW; ++i) {
+    if (i >= vtv) break;
+    wf[0][i] = load_w(0, i);
+    wf[1][i] = load_w(1, i);
+  }
+  for (int b = 0; b * HS < S; ++b) {
+    // the block's direct loads have landed: 2 vtv weight loads or more are younger
+    if (vtv == VTW)
+      wait_vmcnt<2 * VTW>();
+    else if (vtv == VTW - 1)
+      wait_vmcnt<2 * (VTW - 1)>();
+    else
       wait_vmcnt<0>();
-    }
-    __syncthreads();                   // every wave's stage-v loads have landed; slot (v + 2) % 3 is free
-    if (v + 2 < S) issue(v + 2);
-    const uint8_t* base = smem + (v % NBW) * SBW;
-    bf16x8 hf[MTL];
+    __syncthreads();  // in every wave; and block b - 1 is read, so its half is free
+    if ((b + 1) * HS < S) issue_h(b + 1);
+    const uint8_t* base = smem + (b & 1) * HBW;
+    const int end = min((b + 1) * HS, S);
+#pragma unroll 1
+    for (int v = b * HS; v < end; v += 2) {
 #pragma unroll
-    for (int j = 0; j < MTL; ++j) hf[j] = *reinterpret_cast<const bf16x8*>(base + WBW + 16 * j * RB + fro);
+      for (int p = 0; p < 2; ++p) {
+        const uint32_t c0 = (uint32_t)(((v + p) & (HS - 1)) * 4 + g4);
+        bf16x8 hf[MTL];
 #pragma unroll
-    for (int i = 0; i < VTW; ++i) {
-      if (i >= vtv) break;
-      const bf16x8 wf = *reinterpret_cast<const bf16x8*>(base + (VTW * 16 * w + 16 * i) * RB + fro);
+        for (int j = 0; j < MTL; ++j)
+          hf[j] = *reinterpret_cast<const bf16x8*>(base + (16 * j + l16) * HRB + ((c0 ^ (uint32_t)l16) << 4));
 #pragma unroll
-      for (int j = 0; j < MTL; ++j) acc[i][j] = mfma16(wf, hf[j], acc[i][j]);
+        for (int i = 0; i < VTW; ++i) {
+          if (i >= vtv) break;
+#pragma unroll
+          for (int j = 0; j < MTL; ++j) acc[i][j] = mfma16(wf[p][i], hf[j], acc[i][j]);
+          if (p == 1) {
+            wf[0][i] = load_w(v + 2, i);
+            wf[1][i] = load_w(v + 3, i);
+          }
+        }
+      }
     }
   }
-  // C register r of accumulator (i, j): weight row 80 w + 16 i + 4 g4 + r of the range, drafted row 16 j + l16
+  // C register r of accumulator (i, j): weight row 16 (t0 + i) + 4 g4 + r of the range, drafted row 16 j + l16
 #pragma unroll
   for (int j = 0; j < MTL; ++j) {
     const int m = 16 * j + l16;
     if (m >= a.M) continue;
     uint16_t* orow = a.out + (int64_t)m * a.out_stride + R0;
 #pragma unroll
-    for (int i = 0; i < VTW; ++i) {
-      const int n = VTW * 16 * w + 16 * i + 4 * g4;
-      const f32x4 c = acc[i][j];
-      const u32x2 pk = {__builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2){c[0], c[1]}, bf16x2)),
-                        __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2){c[2], c[3]}, bf16x2))};
-      if (n + 4 <= rows) {
-        *reinterpret_cast<u32x2*>(orow + n) = pk;
-      } else {
+    for (int i = 0; i < VTW; ++i)
+      if (i < vtv) store4(orow, 16 * (t0 + i) + 4 * g4, rows, acc[i][j]);
+  }
+}
+
+// ---- K-split form: a workgroup of four waves takes 16 VT weight rows against all of the launch's drafted rows (up to
+//      16 MTL), each wave a quarter of k, the 64-k chunks w, w + 4, ..; the four partial sums meet in LDS and are added
+//      in wave order. Nothing is shared before that, so no wave waits for another: both operands go straight to
+//      registers (whole 128-byte lines, as in the wide form), one chunk ahead.
+//      It pays where the drafted rows, read by every workgroup from L2, are few next to the weight, and where the
+//      other forms have fewer tiles than waves and walk all of k in series: 8192 x 2560 weight rows x hidden, 120
+//      drafted rows 34.8 (pass form) -> 26.6 us, 60 rows 33.3 -> 17.3, 15 rows 32.6 -> 14.7; 40000 x 2560, 15 rows
+//      66 -> 43; 151936 x 2560, 15 rows 145.6 -> 139 (5.6 TB/s).
+namespace ksplit {
+constexpr int NW = 4;
+constexpr int NTH = NW * 64;
+constexpr int KC = 64;                   // k per chunk
+}  // namespace ksplit
+
+template <int VT, int MTL>
+__global__ __launch_bounds__(ksplit::NTH) __attribute__((amdgpu_waves_per_eu(2, 2))) void draft_head_ksplit_kernel(
+    HeadArgs a) {
+  using namespace ksplit;
+  constexpr int TT = VT * MTL;  // tiles: 1 KB of partial sums each per wave
+  __shared__ f32x4 part[NW * TT * 64];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int R0 = blockIdx.x * (16 * VT);
+  const int rows = min(16 * VT, a.N - R0);
+  const int K = a.K, P = K / KC;
+  const int l16 = lane & 15, g4 = lane >> 4;
+  const int last = (rows + 15) / 16 - 1;  // tiles past the last read it again and are not stored
+  const __amdgpu_buffer_rsrc_t rw = buffer_of(a.w + (int64_t)R0 * K, (uint32_t)rows * (uint32_t)K * 2u);
+  const __amdgpu_buffer_rsrc_t rh = buffer_of(a.hidden, 0xFFFFFFFFu);  // (offsets are of rows below M only)
+  const uint32_t woff = ((uint32_t)l16 * (uint32_t)K + 8u * g4) * 2u;
+  const uint32_t tstep = 32u * (uint32_t)K;
+  uint32_t hoff[MTL];
 #pragma unroll
-        for (int e = 0; e < 4; ++e)
-          if (n + e < rows) orow[n + e] = (uint16_t)(pk[e >> 1] >> (16 * (e & 1)));
-      }
+  for (int j = 0; j < MTL; ++j) hoff[j] = drafted_off(a, 16 * j + l16) + 16u * g4;
+  f32x4 acc[VT][MTL];
+#pragma unroll
+  for (int i = 0; i < VT; ++i)
+#pragma unroll
+    for (int j = 0; j < MTL; ++j) acc[i][j] = (f32x4){};
+  bf16x8 wf[2][2][VT], hf[2][2][MTL];
+  auto load = [&](int s, int p) __attribute__((always_inline)) {
+    const uint32_t kb = (uint32_t)p * (KC * 2);
+#pragma unroll
+    for (int i = 0; i < VT; ++i)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) wf[s][h][i] = buffer_load8(rw, woff, (uint32_t)min(i, last) * tstep + kb + 64 * h);
+#pragma unroll
+    for (int j = 0; j < MTL; ++j)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) hf[s][h][j] = buffer_load8(rh, hoff[j], kb + 64 * h);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  auto products = [&](int s) __attribute__((always_inline)) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int i = 0; i < VT; ++i)
+#pragma unroll
+        for (int j = 0; j < MTL; ++j) acc[i][j] = mfma16(wf[s][h][i], hf[s][h][j], acc[i][j]);
+  };
+  if (w < P) load(0, w);
+  for (int p = w; p < P; p += 2 * NW) {
+    if (p + NW < P) load(1, p + NW);
+    products(0);
+    if (p + NW < P) {
+      if (p + 2 * NW < P) load(0, p + 2 * NW);
+      products(1);
     }
   }
+#pragma unroll
+  for (int i = 0; i < VT; ++i)
+#pragma unroll
+    for (int j = 0; j < MTL; ++j) part[(w * TT + i * MTL + j) * 64 + lane] = acc[i][j];
+  __syncthreads();
+  for (int t = w; t < TT; t += NW) {
+    const int i = t / MTL, m = 16 * (t % MTL) + l16;
+    f32x4 c = part[t * 64 + lane];
+#pragma unroll
+    for (int x = 1; x < NW; ++x) {
+      const f32x4 d = part[(x * TT + t) * 64 + lane];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) c[e] += d[e];
+    }
+    if (m < a.M) store4(a.out + (int64_t)m * a.out_stride + R0, 16 * i + 4 * g4, rows, c);
+  }
+}
+
+template <int VT, int MTL>
+void launch_ksplit(const HeadArgs& a, hipStream_t stream) {
+  hipLaunchKernelGGL((draft_head_ksplit_kernel<VT, MTL>), dim3((a.N + 16 * VT - 1) / (16 * VT)), dim3(ksplit::NTH), 0,
+                     stream, a);
+}
+// Rows of the most loaded CU when N rows go out in workgroups of 16 vt.
+int64_t cu_rows(int N, int vt, int cus) {
+  const int64_t wgs = ((int64_t)N + 16 * vt - 1) / (16 * vt);
+  return (wgs + cus - 1) / cus * (16 * vt);
+}
+// The tile height that leaves the most loaded CU fewer rows; the taller where they are even (each workgroup reads the
+// drafted rows once): 40000 rows x 2560, 15 drafted: 43 us with 64-row workgroups, 51 with 128; 32000: 31.5 and 30.7.
+template <int VT, int MTL>
+void launch_ksplit_tall_or_half(const HeadArgs& a, int cus, hipStream_t stream) {
+  if (cu_rows(a.N, VT, cus) <= cu_rows(a.N, VT / 2, cus))
+    launch_ksplit<VT, MTL>(a, stream);
+  else
+    launch_ksplit<VT / 2, MTL>(a, stream);
 }
 
 }  // namespace
@@ -422,31 +553,55 @@ static int draft_head_gemm(const uint16_t* hidden, int64_t row_stride, int rows_
                          "%s: drafted rows and weight need 16-byte alignment, output rows 8-byte alignment "
                          "(row_stride=%lld group_stride=%lld out_stride=%lld)",
                          who, (long long)row_stride, (long long)group_stride, (long long)out_stride);
+  const int cus = mfd_num_cus();
   // one workgroup per CU (128 KB of LDS each), at least 128 weight rows each
-  const int nwg = std::max(1, std::min(mfd_num_cus(), (N + PT - 1) / PT));
-  const int64_t maxrows = (int64_t)N / nwg + 8;
-  if (maxrows * K * 2 >= ((int64_t)1 << 32) ||
+  int nwg = std::max(1, std::min(cus, (N + PT - 1) / PT));
+  if (((int64_t)N / nwg + 8) * K * 2 >= ((int64_t)1 << 32) ||
       ((int64_t)(M - 1) / rows_per_group * group_stride + (int64_t)rows_per_group * row_stride + K) * 2 >=
           ((int64_t)1 << 32))
     return mfd_set_error(MFD_ERR_UNSUPPORTED, "%s: N=%d K=%d M=%d too large for 32-bit offsets", who, N, K, M);
+  // the wide form holds at most wide::WRMAX rows: longer ranges are cut again, to whole rounds of the CUs (one round of
+  // the pass form reads the drafted rows eight times at 248320 x 2560: 313 us, two rounds so: 265)
+  while (N / nwg + 8 > wide::WRMAX) nwg += cus;
+  const int vtw = (N / nwg + 8 + 16 * wide::NW - 1) / (16 * wide::NW);  // tiles of a wave of the wide form
   {
     // the kernels' dynamic LDS limits, raised once per device
     int rc = mfd_set_max_lds(reinterpret_cast<const void*>(&draft_head_kernel), SMEM);
-    if (rc == MFD_OK) rc = mfd_set_max_lds(reinterpret_cast<const void*>(&draft_head_wide_kernel), wide::SMEMW);
+    if (rc == MFD_OK) rc = mfd_set_max_lds(reinterpret_cast<const void*>(&draft_head_wide_kernel<2>), wide::SMEMW);
+    if (rc == MFD_OK) rc = mfd_set_max_lds(reinterpret_cast<const void*>(&draft_head_wide_kernel<3>), wide::SMEMW);
+    if (rc == MFD_OK) rc = mfd_set_max_lds(reinterpret_cast<const void*>(&draft_head_wide_kernel<4>), wide::SMEMW);
+    if (rc == MFD_OK) rc = mfd_set_max_lds(reinterpret_cast<const void*>(&draft_head_wide_kernel<5>), wide::SMEMW);
     if (rc != MFD_OK) return rc;
   }
-  // workgroup ranges of more than two 128-row passes (and at most wide::WRMAX rows): the wide form, which streams
-  // the drafted rows once per workgroup instead of once per pass
-  const bool wide_form = maxrows > 2 * PT && maxrows <= wide::WRMAX;
+  const hipStream_t st = static_cast<hipStream_t>(stream);
   // one launch per 128 drafted rows (each streams the weight once)
   for (int m0 = 0; m0 < M; m0 += MT) {
     HeadArgs a{hidden, row_stride, group_stride, rows_per_group, m0, weight, out + (int64_t)m0 * out_stride,
-               out_stride, std::min(MT, M - m0), N, K, nwg};
-    if (wide_form)
-      hipLaunchKernelGGL(draft_head_wide_kernel, dim3(nwg), dim3(wide::NTH), wide::SMEMW,
-                         static_cast<hipStream_t>(stream), a);
+                out_stride, std::min(MT, M - m0), N, K, nwg};
+    // The form (us at hidden 2560): k-split with up to 32 drafted rows at any vocabulary (28 rows: 32.5 against 36.6
+    // in the pass form at 32000, 146.7 against 146.9 in the wide one at 151936), with up to 64 where a CU gets at most
+    // 64 vocabulary rows (60 rows: 17.3 against 33.3 at 8192, 44.9 against 38.6 at 32000), with more where it gets at
+    // most 32 (120 rows: 26.6 against 34.9 at 8192; 72 against 49.5 at 10000 x 4096): beyond, its reads of the
+    // drafted rows outweigh the weight's. Else the pass form up to 128 rows per CU (32000: 41 against 49 in the wide
+    // form) and the wide form above (34000: 51 against 72, 90000: 101 against 107).
+    if (a.M <= 16)
+      launch_ksplit_tall_or_half<8, 1>(a, cus, st);
+    else if (a.M <= 32)
+      launch_ksplit_tall_or_half<8, 2>(a, cus, st);
+    else if (a.M <= 64 && N <= 64 * cus)
+      launch_ksplit_tall_or_half<4, 4>(a, cus, st);
+    else if (N <= 32 * cus)
+      launch_ksplit_tall_or_half<2, 8>(a, cus, st);
+    else if (N <= PT * cus)
+      hipLaunchKernelGGL(draft_head_kernel, dim3(nwg), dim3(NT), SMEM, st, a);
+    else if (vtw <= 2)
+      hipLaunchKernelGGL(draft_head_wide_kernel<2>, dim3(nwg), dim3(wide::NTH), wide::SMEMW, st, a);
+    else if (vtw == 3)
+      hipLaunchKernelGGL(draft_head_wide_kernel<3>, dim3(nwg), dim3(wide::NTH), wide::SMEMW, st, a);
+    else if (vtw == 4)
+      hipLaunchKernelGGL(draft_head_wide_kernel<4>, dim3(nwg), dim3(wide::NTH), wide::SMEMW, st, a);
     else
-      hipLaunchKernelGGL(draft_head_kernel, dim3(nwg), dim3(NT), SMEM, static_cast<hipStream_t>(stream), a);
+      hipLaunchKernelGGL(draft_head_wide_kernel<5>, dim3(nwg), dim3(wide::NTH), wide::SMEMW, st, a);
     MFD_CHECK_LAUNCH();
   }
   return MFD_OK;

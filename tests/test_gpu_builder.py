@@ -405,8 +405,9 @@ def test_draft_head_gemm_shapes(M, N, K, L, gap):
     """mfd_draft_head_gemm (the LM-head product of DDTreeDraftTopK, P:1523-1532) on ragged shapes: drafted rows
     read in place from [blocks, L, K + gap] hidden states (the anchor row of each block skipped), vocabularies
     that are not multiples of the 128-row pass, more than 128 drafted rows (two launches), and K down to one
-    64-wide stage; the columns past N and the rows past M stay untouched. Vocabularies above 256 rows per
-    workgroup (90000 and up) take the wide form (every workgroup's whole range against k streamed once)."""
+    64-wide stage; the columns past N and the rows past M stay untouched. Vocabularies above 128 rows per CU (33333
+    and up) with more than 32 drafted rows take the wide form (every workgroup's whole range against k streamed
+    once), up to 32 drafted rows the k-split form."""
     import mfd_hip
 
     print(f"case: draft head gemm M={M} N={N} K={K} L={L} gap={gap}", flush=True)
@@ -422,6 +423,39 @@ def test_draft_head_gemm_shapes(M, N, K, L, gap):
     torch.cuda.synchronize()
     hs = hid.view(blocks, L, ld)[:, 1:, :K].reshape(-1, K)[:M]
     _gemm_reference_check(out[:M, :N], hs, w)
+    assert bool((out[:M, N:] == -7.0).all()) and bool((out[M] == -7.0).all())
+
+
+# M on both sides of the tile counts of the k-split form; N on both sides of 32, 64 and 128 rows per CU (256 CUs), of a
+# wave's 2, 3, 4 and 5 tiles in the wide form and of its 640 rows; K of one chunk, of fewer and more chunks than waves,
+# and of a drafted block of the wide form with and without a remainder
+@pytest.mark.parametrize("M,N,K", [(1, 9, 64), (16, 5003, 320), (17, 8200, 192), (32, 40004, 576), (16, 40001, 512),
+                                   (33, 8192, 832), (64, 8200, 256), (64, 16384, 64), (65, 4099, 448), (128, 8192, 512),
+                                   (65, 8193, 320), (64, 16392, 128), (128, 32768, 64), (128, 32776, 256),
+                                   (65, 63500, 320), (33, 63700, 512), (120, 96200, 64), (40, 96300, 192),
+                                   (129, 128900, 320), (33, 129100, 256), (120, 161700, 576), (60, 161900, 64),
+                                   (34, 330000, 128)])
+def test_draft_head_gemm_forms(M, N, K):
+    """mfd_draft_head_gemm at the edges of its forms and of their tiles: the first and last columns and sampled ones
+    against the exact product, every logit finite, the columns past N and the rows past M untouched."""
+    import mfd_hip
+
+    print(f"case: draft head gemm forms M={M} N={N} K={K}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(M * 7 + N + K)
+    L = 8
+    blocks = (M + L - 2) // (L - 1)
+    hid = torch.randn(blocks * L, K, generator=g, device="cuda").to(torch.bfloat16)
+    w = (torch.randn(N, K, generator=g, device="cuda") * 0.05).to(torch.bfloat16)
+    ostride = (N + 3) // 4 * 4 + 4
+    out = torch.full((M + 1, ostride), -7.0, dtype=torch.bfloat16, device="cuda")
+    mfd_hip.call("mfd_draft_head_gemm", hid.data_ptr() + K * 2, K, L - 1, L * K, w.data_ptr(), M, N, K,
+                 out.data_ptr(), ostride, mfd_hip.stream_of(out))
+    torch.cuda.synchronize()
+    sample = torch.randperm(N, generator=torch.Generator().manual_seed(5))[:3000]
+    cols = torch.cat([torch.arange(min(N, 700)), torch.arange(max(0, N - 700), N), sample]).unique().cuda()
+    hs = hid.view(blocks, L, K)[:, 1:].reshape(-1, K)[:M]
+    _gemm_reference_check(out[:M][:, cols], hs, w[cols])
+    assert bool(torch.isfinite(out[:M, :N].float()).all())
     assert bool((out[:M, N:] == -7.0).all()) and bool((out[M] == -7.0).all())
 
 
