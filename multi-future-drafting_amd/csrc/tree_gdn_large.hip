@@ -286,13 +286,31 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(6, 6))) voi
 //                            value columns) lies here
 //   ru   [nml][rs] f32       R rows of the workgroup's value columns, then u rows
 //   path [nml][MAXD] u16, g [nml] f32, beta [nml] f32, depth [nml] i32
+// Two workgroups per CU (two; at most TWO_NODES nodes, 81,600 B at 272 and CT 2, of 81,920): the S0 slice lies where R
+// comes later, T goes over the a_i (all of them read by then), and the R / u rows have no padding; their 16-column
+// halves change places with bit 1 of the row instead, so that four neighbouring rows still fall in different banks.
+constexpr int TWO_NODES = 272;
 struct LargeLds {
   int ts, rs, ss;
   uint32_t kq, t, ru, path, g, beta, dep, total;
 };
-__host__ __device__ inline LargeLds large_lds(int nml, int ct) {
+__host__ __device__ constexpr LargeLds large_lds(int nml, int ct, bool two) {
   LargeLds L{};
   const int cw = 16 * ct;
+  if (two) {
+    L.ts = 2 * MAXD;
+    L.rs = cw;
+    L.ss = cw + 2;
+    L.kq = L.t = 0;
+    L.ru = (uint32_t)nml * 2 * MAXD * 4;
+    const uint32_t rbytes = (uint32_t)nml * L.rs * 4, sbytes = (uint32_t)D * L.ss * 4;
+    L.path = L.ru + (rbytes > sbytes ? rbytes : sbytes);
+    L.g = L.path + (uint32_t)nml * MAXD * 2;
+    L.beta = L.g + (uint32_t)nml * 4;
+    L.dep = L.beta + (uint32_t)nml * 4;
+    L.total = L.dep + (uint32_t)nml * 4;
+    return L;
+  }
   for (int pad = 1; pad >= 0; --pad) {
     L.ts = MAXD + 4 * pad;
     L.rs = cw + 4 * pad;
@@ -310,6 +328,7 @@ __host__ __device__ inline LargeLds large_lds(int nml, int ct) {
   }
   return L;
 }
+static_assert(large_lds(TWO_NODES, 2, true).total <= 80u * 1024u, "two workgroups per CU");
 // Hand-over words of the one-launch form, per (request, key head) group: [0] the group's call count, [1] its
 // workgroups done with this call's Gram rows, [2 + c] the tag of Gram unit c once it is written (call count + 1,
 // and the writer's XCD). A library array (512 KiB), zero at load, in GSYNC_SLOTS sets: each stream that runs the
@@ -337,7 +356,6 @@ __device__ __forceinline__ void gram_rows_to_lds(const GdnLargeArgs& a, int ns, 
 }
 
 constexpr int LT = 512;  // threads of the main kernel: one per node in phase T
-constexpr int PRE = 2;   // 16-node tiles whose K / Q rows and v are requested before phase T
 
 // One workgroup per (request, value head, CW = 16 CT value columns), eight waves; wave w owns the 16-node tiles
 // t = w, w + 8, ... of the R, U and O phases, for all CT 16-column tiles.
@@ -356,16 +374,22 @@ constexpr int PRE = 2;   // 16-node tiles whose K / Q rows and v are requested b
 //   U  u_i = sum_{s < depth} T_i[s] R_path(i,s) (16-byte gathers; registers, then over R in LDS)
 //   O  o_i = E_i + sum_{s < depth} p_i[s] u_path(i,s); u and o leave as 16-byte stores
 // ONE: the one-launch form (a.gsync set); a separate instantiation, so that the two-kernel form keeps its registers
-template <int NMAX, int CT, bool ONE>
-__global__ __launch_bounds__(LT) void tree_gdn_large_kernel(GdnLargeArgs a, int nml) {
+// TWO: two workgroups per CU, for grids of more than one round and trees of at most TWO_NODES nodes. The phases wait on
+// memory, on the serial chain of T and on the stores in turn (VALU 45 % busy, waves waiting 53 % of their time), and one
+// resident workgroup leaves the CU idle meanwhile. So half the LDS (large_lds) and at most 128 registers: the S0
+// fragments are read after T, and tiles are requested one ahead and after T. 4 x 257 nodes, H 32: 35.8 -> 33.0 us;
+// two layers with the context, 8 x 130: 97.4 -> 86.8, one 257-node tree with H 48 (16 columns): 71.0 -> 59.8.
+// Longer trees keep one workgroup per CU.
+template <int NMAX, int CT, bool ONE, bool TWO>
+__global__ __launch_bounds__(LT) __attribute__((amdgpu_waves_per_eu(TWO ? 4 : 2))) void tree_gdn_large_kernel(GdnLargeArgs a, int nml) {
   constexpr int CW = 16 * CT;                 // value columns of a workgroup
-  constexpr int MAXT = (NMAX / 16 + 7) / 8;   // 16-node tiles per wave at most
+  constexpr int MAXT = ((TWO && NMAX > TWO_NODES ? TWO_NODES : NMAX) / 16 + 7) / 8;  // 16-node tiles per wave at most
   extern __shared__ __align__(16) uint8_t lds[];
-  const LargeLds L = large_lds(nml, CT);
+  const LargeLds L = large_lds(nml, CT, TWO);
   const int TS = L.ts, RS = L.rs, SS = L.ss;
   float* const KQ = reinterpret_cast<float*>(lds + L.kq);
   float* const TT = reinterpret_cast<float*>(lds + L.t);
-  float* const S0L = reinterpret_cast<float*>(lds + L.t);
+  float* const S0L = reinterpret_cast<float*>(lds + (TWO ? L.ru : L.t));
   float* const RU = reinterpret_cast<float*>(lds + L.ru);
   uint16_t* const PT = reinterpret_cast<uint16_t*>(lds + L.path);
   float* const Gs = reinterpret_cast<float*>(lds + L.g);
@@ -377,6 +401,11 @@ __global__ __launch_bounds__(LT) void tree_gdn_large_kernel(GdnLargeArgs a, int 
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int g4 = lane >> 4;
   const int l16 = lane & 15;
+  constexpr int PRE = TWO ? 1 : 2;  // 16-node tiles whose K / Q rows and v are in registers or on their way
+  // row i, columns 16 ct + c .. of the R / u rows
+  auto ru = [&](int i, int ct, int c) __attribute__((always_inline)) -> float* {
+    return TWO ? &RU[i * CW + 16 * (CT == 2 ? ct ^ ((i >> 1) & 1) : ct) + c] : &RU[i * RS + 16 * ct + c];
+  };
 
   // workgroup -> (request, key head, value head member x column group); the sub-units of one (request, key head)
   // land on one XCD (workgroup id modulo 8), so its q / k rows and Gram rows come from that XCD's L2 after the first
@@ -487,9 +516,24 @@ __global__ __launch_bounds__(LT) void tree_gdn_large_kernel(GdnLargeArgs a, int 
   const __amdgpu_buffer_rsrc_t rs_v = rsrc(a.v + ((size_t)ns * a.H + h) * D, (uint32_t)n * HD * 2);
   const int tn = 4 * g4 + (l16 & 3);      // node of this lane within a tile (transposed layout)
   const int tc = 4 * (l16 >> 2);          // first of this lane's four columns within a 16-column tile
-  u32x4 fk[2][D / 32], fq[2][D / 32];
-  u32x2 vv[2][CT];
+  u32x4 fk[PRE][D / 32], fq[PRE][D / 32];
+  u32x2 vv[PRE][CT];
   auto load_tile = [&](int t, int slot) __attribute__((always_inline)) {
+    if constexpr (TWO) {
+      // the tile in the scalar offset (fewer registers), which the buffers' bounds check needs inside the buffer
+      if (t >= nt16) return;
+      const uint32_t sk = (uint32_t)(16 * t * HKD) * 2u, sv = (uint32_t)(16 * t * HD) * 2u;
+      const uint32_t ok = (uint32_t)(l16 * HKD + 8 * g4) * 2u, ov = (uint32_t)(tn * HD + cb + tc) * 2u;
+#pragma unroll
+      for (int kc = 0; kc < D / 32; ++kc) {
+        fk[slot][kc] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rs_k, ok, sk + kc * 64, 0));
+        fq[slot][kc] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rs_q, ok, sk + kc * 64, 0));
+      }
+#pragma unroll
+      for (int ct = 0; ct < CT; ++ct)
+        vv[slot][ct] = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(rs_v, ov, sv + 32 * ct, 0));
+      return;
+    }
     const uint32_t off = (uint32_t)((16 * t + l16) * HKD + 8 * g4) * 2u;
 #pragma unroll
     for (int kc = 0; kc < D / 32; ++kc) {
@@ -504,6 +548,7 @@ __global__ __launch_bounds__(LT) void tree_gdn_large_kernel(GdnLargeArgs a, int 
   __syncthreads();
   // S0 B fragments of this wave's column tiles: column cb + 16 ct + l16, k = 32 kc + 8 g4 .. + 7
   bf16x8 sb[CT][D / 32];
+  auto read_s0 = [&]() __attribute__((always_inline)) {
 #pragma unroll
   for (int ct = 0; ct < CT; ++ct)
 #pragma unroll
@@ -515,6 +560,8 @@ __global__ __launch_bounds__(LT) void tree_gdn_large_kernel(GdnLargeArgs a, int 
         pk[e] = __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2){src[(2 * e) * SS], src[(2 * e + 1) * SS]}, bf16x2));
       sb[ct][kc] = __builtin_bit_cast(bf16x8, pk);
     }
+  };
+  if constexpr (!TWO) read_s0();
 
   if (fused) {
     __syncthreads();  // every wave has its S0 fragments: the T region is free again (scratch of a local chunk)
@@ -583,20 +630,21 @@ __global__ __launch_bounds__(LT) void tree_gdn_large_kernel(GdnLargeArgs a, int 
     }
     *reinterpret_cast<f32x4*>(&KQ[i * 2 * MAXD + 4 * c]) = xv;
   }
-  // the first tiles' K / Q rows and v, in flight during T: waves 0-3 (the T threads of the first 256 nodes) request
+  // (one workgroup per CU) the first tiles' K / Q rows and v, in flight during T: waves 0-3 (the T threads of the first 256 nodes) request
   // theirs before the barrier, the others after it, where their issue (a wave waits there for room in the CU's
   // load queue) runs beside T instead of holding the barrier
-  if (w < 4) {
+  if (!TWO && w < 4) {
 #pragma unroll
     for (int j = 0; j < PRE; ++j) load_tile(w + 8 * j, j);
   }
   __syncthreads();  // coefficients complete; the S0 slice is dead (phase T writes over it)
-  if (w >= 4) {
+  if (!TWO && w >= 4) {
 #pragma unroll
     for (int j = 0; j < PRE; ++j) load_tile(w + 8 * j, j);
   }
 
   // ---- phase T: T_i[d-1] = 1, T_i[s] = -sum_{m>s} T_i[m] a_{path(m)}[s] (right-looking over m)
+  float Tr[MAXD];
   if (tid < n) {
     const int i = tid;
     const int d = DP[i];
@@ -607,7 +655,7 @@ __global__ __launch_bounds__(LT) void tree_gdn_large_kernel(GdnLargeArgs a, int 
 #pragma unroll
       for (int e = 0; e < 4; ++e) pth[s4 + e] = (int)((pp[e >> 1] >> (16 * (e & 1))) & 0xFFFFu);
     }
-    float acc[MAXD], Tr[MAXD];
+    float acc[MAXD];
 #pragma unroll
     for (int s = 0; s < MAXD; ++s) acc[s] = 0.f;
 #pragma unroll
@@ -625,9 +673,20 @@ __global__ __launch_bounds__(LT) void tree_gdn_large_kernel(GdnLargeArgs a, int 
         }
       }
     }
+  }
+  if constexpr (TWO) {
+    read_s0();
+    __syncthreads();  // the a_i and the S0 slice are read: T and R go over them
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  if (tid < n) {
 #pragma unroll
     for (int s = 0; s < MAXD; s += 4)
-      *reinterpret_cast<f32x4*>(&TT[i * TS + s]) = (f32x4){Tr[s], Tr[s + 1], Tr[s + 2], Tr[s + 3]};
+      *reinterpret_cast<f32x4*>(&TT[tid * TS + s]) = (f32x4){Tr[s], Tr[s + 1], Tr[s + 2], Tr[s + 3]};
+  }
+  if constexpr (TWO) {
+    __builtin_amdgcn_sched_barrier(0);
+    load_tile(w, 0);
   }
 
   // ---- phase R (no barrier before it: R writes only the ru region and reads the gates)
@@ -636,7 +695,8 @@ __global__ __launch_bounds__(LT) void tree_gdn_large_kernel(GdnLargeArgs a, int 
   for (int j = 0; j < MAXT; ++j) {
     const int t = w + 8 * j;
     if (t >= nt16) break;
-    const int slot = j & 1;
+    if (TWO) __builtin_amdgcn_sched_barrier(0);
+    const int slot = j & (PRE - 1);
     const int i = 16 * t + tn;
     const float eg = __expf(Gs[i]);
     const float bi = Bs[i];
@@ -660,9 +720,9 @@ __global__ __launch_bounds__(LT) void tree_gdn_large_kernel(GdnLargeArgs a, int 
         rv[e] = bi * (vf[e] - eg * kt[e]);
         E[j][ct][e] = eg * qt[e];
       }
-      *reinterpret_cast<f32x4*>(&RU[i * RS + 16 * ct + tc]) = rv;
+      *reinterpret_cast<f32x4*>(ru(i, ct, tc)) = rv;
     }
-    if (j + 2 < MAXT && t + 16 < nt16) load_tile(t + 16, slot);
+    if (j + PRE < MAXT && t + 8 * PRE < nt16) load_tile(t + 8 * PRE, slot);
   }
   __syncthreads();  // T rows and R rows complete
 
@@ -677,6 +737,7 @@ __global__ __launch_bounds__(LT) void tree_gdn_large_kernel(GdnLargeArgs a, int 
     const int d = DP[i];
 #pragma unroll
     for (int ct = 0; ct < CT; ++ct) U[j][ct] = (f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll(TWO ? 1 : MAXD / 4)
     for (int s4 = 0; s4 < MAXD; s4 += 4) {
       if (__builtin_amdgcn_ballot_w64(s4 < d) == 0) break;
       const u32x2 pp = *reinterpret_cast<const u32x2*>(&PT[i * MAXD + s4]);
@@ -688,7 +749,7 @@ __global__ __launch_bounds__(LT) void tree_gdn_large_kernel(GdnLargeArgs a, int 
         const float wt = on ? tv[q] : 0.f;
 #pragma unroll
         for (int ct = 0; ct < CT; ++ct) {
-          const f32x4 rv = *reinterpret_cast<const f32x4*>(&RU[jn * RS + 16 * ct + tc]);
+          const f32x4 rv = *reinterpret_cast<const f32x4*>(ru(jn, ct, tc));
 #pragma unroll
           for (int e = 0; e < 4; ++e) U[j][ct][e] = fmaf(wt, rv[e], U[j][ct][e]);
         }
@@ -701,7 +762,7 @@ __global__ __launch_bounds__(LT) void tree_gdn_large_kernel(GdnLargeArgs a, int 
     const int t = w + 8 * j;
     if (t >= nt16) break;
 #pragma unroll
-    for (int ct = 0; ct < CT; ++ct) *reinterpret_cast<f32x4*>(&RU[(16 * t + tn) * RS + 16 * ct + tc]) = U[j][ct];
+    for (int ct = 0; ct < CT; ++ct) *reinterpret_cast<f32x4*>(ru(16 * t + tn, ct, tc)) = U[j][ct];
   }
   __syncthreads();  // u rows complete
 
@@ -714,6 +775,7 @@ __global__ __launch_bounds__(LT) void tree_gdn_large_kernel(GdnLargeArgs a, int 
     if (t >= nt16) break;
     const int i = 16 * t + tn;
     const int d = DP[i];
+#pragma unroll(TWO ? 1 : MAXD / 4)
     for (int s4 = 0; s4 < MAXD; s4 += 4) {
       if (__builtin_amdgcn_ballot_w64(s4 < d) == 0) break;
       const u32x2 pp = *reinterpret_cast<const u32x2*>(&PT[i * MAXD + s4]);
@@ -725,7 +787,7 @@ __global__ __launch_bounds__(LT) void tree_gdn_large_kernel(GdnLargeArgs a, int 
         const float wt = on ? pv[q] : 0.f;
 #pragma unroll
         for (int ct = 0; ct < CT; ++ct) {
-          const f32x4 uv = *reinterpret_cast<const f32x4*>(&RU[jn * RS + 16 * ct + tc]);
+          const f32x4 uv = *reinterpret_cast<const f32x4*>(ru(jn, ct, tc));
 #pragma unroll
           for (int e = 0; e < 4; ++e) E[j][ct][e] = fmaf(wt, uv[e], E[j][ct][e]);
         }
@@ -740,15 +802,15 @@ __global__ __launch_bounds__(LT) void tree_gdn_large_kernel(GdnLargeArgs a, int 
   }
 }
 
-template <int NMAX, int CT, bool ONE>
+template <int NMAX, int CT, bool ONE, bool TWO>
 int run_large_ct(const GdnLargeArgs& a, int nml, hipStream_t s) {
-  const int lds = (int)large_lds(nml, CT).total;
-  if (int rc = mfd_set_max_lds(reinterpret_cast<const void*>(&tree_gdn_large_kernel<NMAX, CT, ONE>), 160 * 1024))
+  const int lds = (int)large_lds(nml, CT, TWO).total;
+  if (int rc = mfd_set_max_lds(reinterpret_cast<const void*>(&tree_gdn_large_kernel<NMAX, CT, ONE, TWO>), 160 * 1024))
     return rc;
   const int P = a.R * a.HK;
   const int SUB = (a.H / a.HK) * (D / (16 * CT));
   const dim3 grid(8 * ((P + 7) / 8) * SUB);
-  hipLaunchKernelGGL((tree_gdn_large_kernel<NMAX, CT, ONE>), grid, dim3(LT), lds, s, a, nml);
+  hipLaunchKernelGGL((tree_gdn_large_kernel<NMAX, CT, ONE, TWO>), grid, dim3(LT), lds, s, a, nml);
   MFD_CHECK_LAUNCH();
   return MFD_OK;
 }
@@ -797,10 +859,10 @@ int run_large(const GdnLargeArgs& a, int max_nodes, hipStream_t s) {
   // 32 value columns per workgroup while that still gives every CU a workgroup (the tree part is then shared by twice
   // the columns) and the LDS allows it; 16 otherwise
   const int cus = mfd_num_cus();
-  const bool wide = (int64_t)a.R * a.H * (D / 32) >= cus && large_lds(nml, 2).total <= 160u * 1024u;
+  const bool wide = (int64_t)a.R * a.H * (D / 32) >= cus && large_lds(nml, 2, false).total <= 160u * 1024u;
   const int ct = wide ? 2 : 1;
   const int SUB = (a.H / a.HK) * (D / (16 * ct));
-  const LargeLds L = large_lds(nml, ct);
+  const LargeLds L = large_lds(nml, ct, false);
   // one launch when the whole grid fits on the CUs at once and each (request, key head) group has a workgroup per
   // Gram chunk: the chunks are then computed inside the main kernel while its phase-0 loads are in flight, instead
   // of by a kernel of their own before it. (With more workgroups than CUs the form still works, a workgroup taking
@@ -815,8 +877,13 @@ int run_large(const GdnLargeArgs& a, int max_nodes, hipStream_t s) {
     hipLaunchKernelGGL(tree_gram_kernel<NMAX>, dim3(8 * P8 * nchunks), dim3(512), 0, s, b, nchunks);
     MFD_CHECK_LAUNCH();
   }
-  if (b.gsync) return wide ? run_large_ct<NMAX, 2, true>(b, nml, s) : run_large_ct<NMAX, 1, true>(b, nml, s);
-  return wide ? run_large_ct<NMAX, 2, false>(b, nml, s) : run_large_ct<NMAX, 1, false>(b, nml, s);
+  if (b.gsync)
+    return wide ? run_large_ct<NMAX, 2, true, false>(b, nml, s) : run_large_ct<NMAX, 1, true, false>(b, nml, s);
+  if (NMAX <= TWO_NODES || nml <= TWO_NODES)
+    return wide ? run_large_ct<NMAX, 2, false, true>(b, nml, s) : run_large_ct<NMAX, 1, false, true>(b, nml, s);
+  if constexpr (NMAX > TWO_NODES)
+    return wide ? run_large_ct<NMAX, 2, false, false>(b, nml, s) : run_large_ct<NMAX, 1, false, false>(b, nml, s);
+  return MFD_OK;
 }
 
 }  // namespace

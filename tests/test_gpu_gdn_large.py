@@ -82,6 +82,24 @@ def test_tree_gdn_large_varlen(sizes, HK, H):
     _check(u, o, d, f"sizes={sizes}")
 
 
+@pytest.mark.parametrize("sizes,HK,H", [
+    ([272, 5, 1, 129, 257, 144], 4, 24),  # the most nodes of two workgroups per CU, 32 columns; fewer tiles than waves
+    ([272, 16, 130, 200, 3], 4, 8),       # the same with 16 columns per workgroup
+    ([256, 131, 17], 8, 24),              # the 256-node layout
+    ([273, 272, 40, 260], 8, 16),         # one node more: one workgroup per CU
+])
+def test_tree_gdn_large_two_per_cu(sizes, HK, H):
+    """Grids of more than one round on 256 CUs (the first three), at the node counts where the form changes."""
+    import tree_gdn_kernel
+
+    d = gdn_inputs(sizes, HK, H, 128, seed=sum(sizes) + H)
+    t = _dev(d)
+    print(f"case: two per CU {sizes} HK={HK} H={H}", flush=True)
+    u, o = tree_gdn_kernel.tree_gdn_varlen(t["q"], t["k"], t["v"], t["g_cum"], t["beta"], t["s0"], t["parents"],
+                                           t["cu_nodes"], max_nodes=max(sizes))
+    _check(u, o, d, f"{sizes}")
+
+
 def test_tree_gdn_large_one_launch_two_streams():
     """Two streams running the one-launch form at once (one 257-node tree each, HK 16 / H 32: 256 workgroups per
     call, so the second call's workgroups start as the first's end): each stream has hand-over words of its own."""
