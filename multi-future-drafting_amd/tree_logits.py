@@ -6,8 +6,8 @@ of exp(x - max) in a fixed order from a table of e^x over bf16 values, and the l
 elements; a second small kernel takes a row's exact top k from the few groups that can hold it. The top-k order
 is value descending, token id ascending (torch.topk leaves ties unspecified), and log Z is reproducible bit for
 bit on the CPU while agreeing with torch.logsumexp to about one fp32 ulp. float32 / float16 logits, which the
-reference also takes, go through csrc/logits_wide.hip: one workgroup per row, an exact radix select on 32-bit
-order keys and an fp32 log Z.
+reference also takes, go through csrc/logits_wide.hip: one workgroup per row, an exact selection on 32-bit order
+keys and an fp32 log Z.
 """
 
 from __future__ import annotations
@@ -26,7 +26,7 @@ def topk_logz(logits: torch.Tensor, k: int, ids_dtype=torch.int64, with_logz: bo
     mfd_topk_logz_workspace_bytes(R, V, k) bytes (both optional, for graph capture without allocation).
     Limits: k <= 256; for bf16 ceil(V / 2048) * max(k, 1) <= 8192 for k <= 32 and ceil(V / 8192) * k <= 8192
     above; larger requests raise MFDError. fp16 / fp32 logits (the reference
-    takes any float dtype) go through a radix-select kernel with an fp32 log Z (no workspace, no V limit)."""
+    takes any float dtype) go through a kernel of their own with an fp32 log Z (no workspace, no V limit)."""
     mfd_hip.require_cuda(logits, vocab_ids)
     wide = {torch.float32: 0, torch.float16: 1}.get(logits.dtype)  # MFD_DTYPE_F32 / MFD_DTYPE_F16
     if logits.dtype != torch.bfloat16 and wide is None:

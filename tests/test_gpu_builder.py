@@ -562,6 +562,54 @@ def test_topk_logz_wide_dtypes(dtype, kind, rows, V, k):
         assert np.abs(got[ok] - lp_ref[ok]).max(initial=0) <= 4e-6 * max(1.0, np.abs(lp_ref[ok]).max(initial=0))
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+@pytest.mark.parametrize("kind,V,k", [("constant", 50000, 256), ("masked", 70001, 64), ("tied2048", 60000, 5),
+                                      ("tied2049", 60000, 5), ("ascending", 40000, 256), ("descending", 9001, 200),
+                                      ("nan", 20000, 8), ("tiny", 300, 256), ("tiny", 5, 5), ("clustered", 33000, 256)])
+def test_topk_logz_wide_selection_edges(dtype, kind, V, k):
+    """The selection of the float32 / float16 rows where its bound holds few elements and where it holds too many for
+    its list (2048): ids in the order (value descending, NaN first, -0 as 0; column ascending) for every row."""
+    import tree_logits
+
+    g = torch.Generator().manual_seed(V + k)
+    x = torch.randn(3, V, generator=g)
+    if kind == "constant":
+        x = torch.full((3, V), 1.5)
+        x[2, ::2] = -0.0
+        x[2, 1::2] = 0.0
+    elif kind == "masked":  # all but 40, 64 and 3000 columns at -inf
+        for r, keep in enumerate((40, 64, 3000)):
+            cols = torch.randperm(V, generator=g)[:keep]
+            row = torch.full((V,), float("-inf"))
+            row[cols] = x[r, cols]
+            x[r] = row
+    elif kind.startswith("tied"):
+        x = x.clamp(max=4.0)
+        for r in range(3):
+            x[r, torch.randperm(V, generator=g)[: int(kind[4:])]] = 9.0
+    elif kind in ("ascending", "descending"):
+        x = torch.sort(x, dim=1, descending=kind == "descending").values
+    elif kind == "nan":
+        x[0, 77] = x[1, 3] = x[1, 19999] = float("nan")
+        x[2, 5] = float("inf")
+    elif kind == "clustered":  # the largest in one thread's vectors
+        x[:, 512 * 16 : 512 * 16 + 8] += 50
+        x[:, : 4] += 50
+    x = x.to(dtype)
+    print(f"case: topk_logz wide selection {dtype} {kind} V={V} k={k}", flush=True)
+    logp, ids, logz = tree_logits.topk_logz(x.cuda(), k, with_logz=True)
+    torch.cuda.synchronize()
+    xv = x.double().numpy() + 0.0  # (-0 + 0 = 0)
+    for r in range(3):
+        order = np.argsort(np.where(np.isnan(xv[r]), -np.inf, -xv[r]), kind="stable")
+        if np.isnan(xv[r]).any():  # NaN before +inf, by column
+            order = np.concatenate([np.flatnonzero(np.isnan(xv[r])), order[~np.isnan(xv[r][order])]])
+        np.testing.assert_array_equal(ids[r].cpu().numpy(), order[:k])
+        ref = torch.logsumexp(x[r].double(), 0).item()
+        lz = logz[r].item()
+        assert (np.isnan(lz) and np.isnan(ref)) or lz == ref or abs(lz - ref) <= 2e-6 * max(1.0, abs(ref))
+
+
 def test_topk_logz_wide_vocab_map_and_api():
     """A reduced vocabulary's id map and the reference's entry points on float32 logits."""
     import tree_logits
