@@ -247,6 +247,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))
   // ---- workgroup -> (request, KV head, split, unit group). A program p = (rank, KV head, split) runs
   //      on XCD p % 8 (workgroup id modulo 8), and its unit groups are consecutive there, so the groups
   //      that read the same K / V run together and share that XCD's L2.
+  const bool fold = CTX != CTX_FLAT && a.fold;
   const int P = a.bs * a.Hkv * a.S;
   const int NG = a.ngroups;
   const int id = blockIdx.x;
@@ -256,7 +257,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))
   if (pidx >= P) return;
   int s, kvh, b;
   int fchunk = 0, fsplits = 1;  // split batch: keys per split of this request and their number
-  if (a.fold) {
+  if (fold) {
     // the splits in use come first, request by request, so that no workgroup waits behind empty ones; the grid has room
     // for SC of every request
     const int j = pidx / a.Hkv;
@@ -340,7 +341,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))
   int lo = 0, hi = ctx;
   int n_blk_tiles = (KL + TK - 1) / TK;
   bool whole = a.S == 1;  // this workgroup sees every key of its queries
-  if (a.fold) {
+  if (fold) {
     lo = s * fchunk;
     hi = min(lo + fchunk, ctx);
     whole = fsplits == 1;
@@ -930,7 +931,7 @@ extern "C" int mfd_mode_attn(const uint16_t* q, int64_t q_st, int64_t q_sh, cons
   a.req_idx = req_idx; a.ctx_lens = ctx_lens; a.ctx_const = ctx_len_const;
   a.out = out; a.o_st = o_st; a.o_sh = o_sh;
   const int64_t rows = (int64_t)bs * H * KL;
-  a.fold = num_ctx_splits > 1 && ctx_lens && bs > 1;
+  a.fold = num_ctx_splits > 1 && ctx_lens && slot_table && bs > 1;  // (flat contexts keep their even splits)
   const int SP = num_ctx_splits > 1 ? num_ctx_splits + (a.fold ? 0 : 1) : 1;
   a.ws_o = reinterpret_cast<uint16_t*>(workspace);
   a.ws_lse = workspace ? reinterpret_cast<float*>(a.ws_o + (int64_t)SP * rows * D) : nullptr;
