@@ -186,8 +186,7 @@ int mfd_gdn_commit(float* state, int64_t state_layer_stride, const float* u, int
  *               page_size + t % page_size (page table). row = req_idx ? req_idx[b] : b (device int64)
  *   ctx_lens    device int64 [bs], or NULL to use ctx_len_const for every request
  *   num_ctx_splits  >= 1; 1 = one pass, > 1 = context split in that many chunks, the block keys in a partial
- *               of their own, and a log-sum-exp merge of the num_ctx_splits + 1 partials; with ctx_lens, chunks of
- *               at least 128 keys, and for bs > 1 at most that many per request, fewer for short ones
+ *               of their own, and a log-sum-exp merge of the num_ctx_splits + 1 partials
  *   out         token t, head h: out + t * o_st + h * o_sh (bf16)
  *   workspace   device scratch of mfd_mode_attn_workspace_bytes(...) bytes (NULL allowed when 0)
  * Requires D == 128 and num_modes * block_size <= 65536 (any num_modes: when K * L is not a multiple of 32

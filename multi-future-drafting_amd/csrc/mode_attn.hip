@@ -35,8 +35,7 @@
 // The running max is rescaled lazily (only when a score exceeds it by more than 2^8), and only the last
 // context tile and the block tiles are masked.
 // The request's block keys are extra 64-key tiles with the mode mask: after the context in a single pass,
-// or as a partial of their own when one request's context is split; in a split batch every request takes the splits its
-// length asks for (split_chunk), the last of them with the block keys, and a request of one split is done. One pass: the normalised output is written as
+// or as a partial of their own when the context is split. One pass: the normalised output is written as
 // bf16. Split: partials (O / l in fp16 with a power-of-two row scale, and lse) go to the workspace and a merge
 // kernel combines them
 // (inference/hf/mode_attention.py:91-117).
@@ -120,9 +119,6 @@ struct AttnArgs {
   int bs, K, L, H, Hkv, G, S, SC, causal;  // S partials per (request, KV head): SC context splits + 1 block
   float scale_log2;
   int ngroups;    // unit groups (of NW units, the kernel's waves) per (request, KV head)
-  int per_cu;     // workgroups a CU holds: 2 of four waves, 1 of eight
-  int slots;      // workgroups the chip holds
-  int fold;       // split batch: a request's last split takes its block keys too, and writes the output if it is the only one
 };
 
 // Combine a value with the one in the other 32-lane half of the wave (lane l and lane l ^ 32 hold the two
@@ -194,34 +190,6 @@ __device__ __forceinline__ int request_of_rank(const int64_t* ctx_lens, int bs, 
   return rho;
 }
 
-// Keys per context split of a request with ctx keys: an even share of SC splits, in whole 64-key tiles, and with lengths
-// on the device (the host, which picks SC, does not know them) no less than 128, below which a split's fixed cost
-// outweighs it, nor, in a batch, than fair_chunk.
-__device__ __forceinline__ int split_chunk(const AttnArgs& a, int ctx, int fair) {
-  int per = (ctx + a.SC - 1) / a.SC;
-  if (a.ctx_lens) per = max(per, 2 * TK);
-  if (a.fold) per = max(per, min(fair, ctx));
-  return max(TK, (per + TK - 1) / TK * TK);
-}
-// What the chip allows a batch: with Q workgroup slots for every (KV head, unit group), chunks of total / (Q - bs) keys
-// start all at once (but no more than 0.8 Q's share is asked for: then a few short ones wait). Slots are counted one per
-// CU, where workgroups of four waves run fastest too, and two only when one would leave no room to split. So long
-// requests are split and short ones are not. (By whole waves.) Auto splits, 8 modes x 16 tokens, before (even splits, as
-// many as cover the CUs) and with it: 11 requests of 85 .. 7215 keys, 16 heads 151 -> 57 us; 14 of 82 .. 8129, 32 heads
-// 308 -> 148; 7 of 105 .. 4197, 40 heads 135 -> 52; 5 of 2000, 32 heads 51 -> 45; 2 of 990 and 3741, 16 heads 31 -> 30.
-__device__ __forceinline__ int fair_chunk(const AttnArgs& a) {
-  int64_t total = 0;
-  for (int b = threadIdx.x & 63; b < a.bs; b += 64) total += a.ctx_lens[b];
-#pragma unroll
-  for (int d = 32; d >= 1; d >>= 1) total += __shfl_xor(total, d);
-  const int teams = a.Hkv * a.ngroups;
-  const int cus = a.slots / a.per_cu;
-  const int64_t wgs = (int64_t)a.bs * teams;
-  const int64_t slots = 4 * wgs <= cus ? cus : a.slots;
-  const int64_t room = max(slots - wgs, slots * 4 / 5);
-  return (int)min(total * teams / room + 1, (int64_t)0x7FFFFFFF);
-}
-
 template <int CTX, int NW>
 __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2, 2))) void mode_attn_kernel(AttnArgs a) {
   static_assert(NW == 4 || NW == 8, "workgroups of 4 or 8 waves");
@@ -247,7 +215,6 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))
   // ---- workgroup -> (request, KV head, split, unit group). A program p = (rank, KV head, split) runs
   //      on XCD p % 8 (workgroup id modulo 8), and its unit groups are consecutive there, so the groups
   //      that read the same K / V run together and share that XCD's L2.
-  const bool fold = CTX != CTX_FLAT && a.fold;
   const int P = a.bs * a.Hkv * a.S;
   const int NG = a.ngroups;
   const int id = blockIdx.x;
@@ -255,58 +222,11 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))
   const int ug = jx % NG;
   const int pidx = (jx / NG) * 8 + (id & 7);
   if (pidx >= P) return;
-  int s, kvh, b;
-  int fchunk = 0, fsplits = 1;  // split batch: keys per split of this request and their number
-  if (fold) {
-    // the splits in use come first, request by request, so that no workgroup waits behind empty ones; the grid has room
-    // for SC of every request
-    const int j = pidx / a.Hkv;
-    kvh = pidx % a.Hkv;
-    const int fair = fair_chunk(a);
-    // more requests than the chip holds at once: longest first (ties by index), which takes a loop over all of them
-    const bool ranked = (int64_t)a.bs * a.Hkv * NG > a.slots;
-    int hit_b = -1, hit_s = 0, base = 0;
-    for (int b0 = 0; b0 < a.bs && hit_b < 0; b0 += 64) {
-      const int own = b0 + lane < a.bs ? (int)a.ctx_lens[b0 + lane] : -1;
-      const int chunk = split_chunk(a, own, fair);
-      const int ns = own >= 0 ? max(1, (own + chunk - 1) / chunk) : 0;
-      int before;  // splits of the requests ahead of this lane's
-      if (ranked) {
-        before = 0;
-        for (int x = 0; x < a.bs; ++x) {
-          const int cx = (int)a.ctx_lens[x];
-          const int kx = split_chunk(a, cx, fair);
-          before += (cx > own || (cx == own && x < b0 + lane)) ? max(1, (cx + kx - 1) / kx) : 0;
-        }
-      } else {
-        int inc = ns;
-#pragma unroll
-        for (int d = 1; d < 64; d <<= 1) {
-          const int o = __shfl_up(inc, d);
-          if (lane >= d) inc += o;
-        }
-        before = base + inc - ns;
-        base += __builtin_amdgcn_readlane(inc, 63);
-      }
-      const uint64_t hit = __builtin_amdgcn_ballot_w64(j >= before && j < before + ns);
-      if (hit) {
-        const int l = __builtin_ctzll(hit);
-        hit_b = b0 + l;
-        hit_s = j - __builtin_amdgcn_readlane(before, l);
-        fchunk = __builtin_amdgcn_readlane(chunk, l);
-        fsplits = __builtin_amdgcn_readlane(ns, l);
-      }
-    }
-    if (hit_b < 0) return;
-    b = hit_b;
-    s = hit_s;
-  } else {
-    s = pidx % a.S;
-    const int bk = pidx / a.S;
-    kvh = bk % a.Hkv;
-    const int rho = bk / a.Hkv;
-    b = __builtin_amdgcn_readfirstlane((a.ctx_lens && a.bs > 1) ? request_of_rank(a.ctx_lens, a.bs, rho) : rho);
-  }
+  const int s = pidx % a.S;
+  const int bk = pidx / a.S;
+  const int kvh = bk % a.Hkv;
+  const int rho = bk / a.Hkv;
+  const int b = __builtin_amdgcn_readfirstlane((a.ctx_lens && a.bs > 1) ? request_of_rank(a.ctx_lens, a.bs, rho) : rho);
 
   const int upr = (KL + UROWS - 1) / UROWS;  // units per query head (the last one padded when KL % 32 != 0)
   const int U = a.G * upr;
@@ -334,22 +254,16 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))
 
   const int ctx = __builtin_amdgcn_readfirstlane(a.ctx_lens ? (int)a.ctx_lens[b] : a.ctx_const);
   const int64_t trow = a.req_idx ? a.req_idx[b] : b;
-  // one pass (S = 1): the whole context, then the block tiles. Split, one request (S = SC + 1 partials): partial
-  // s < SC takes a range of whole context tiles, partial SC only the block tiles (so that the block work is not
-  // added to the critical path of a context split). Split batch (fold, S = SC): ranges of the request's own chunk, the
-  // last one with the block tiles
+  // one pass (S = 1): the whole context, then the block tiles. Split (S = SC + 1 partials): partial s < SC
+  // takes a range of whole context tiles, partial SC only the block tiles (so that the block work is not
+  // added to the critical path of a context split)
   int lo = 0, hi = ctx;
   int n_blk_tiles = (KL + TK - 1) / TK;
-  bool whole = a.S == 1;  // this workgroup sees every key of its queries
-  if (fold) {
-    lo = s * fchunk;
-    hi = min(lo + fchunk, ctx);
-    whole = fsplits == 1;
-    if (s < fsplits - 1) n_blk_tiles = 0;
-  } else if (a.S > 1) {
+  if (a.S > 1) {
     if (s < a.SC) {
-      const int chunk = __builtin_amdgcn_readfirstlane(split_chunk(a, ctx, 0));
-      lo = (int)min((int64_t)s * chunk, (int64_t)ctx);
+      const int per = (ctx + a.SC - 1) / a.SC;
+      const int chunk = max(TK, (per + TK - 1) / TK * TK);
+      lo = min(s * chunk, ctx);
       hi = min(lo + chunk, ctx);
       n_blk_tiles = 0;
     } else {
@@ -358,7 +272,13 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))
   }
   const int n_ctx_tiles = (hi - lo + TK - 1) / TK;
   const int ntiles = n_ctx_tiles + n_blk_tiles;
-  if (ntiles == 0) return;  // an empty split: the merge does not look at it
+  if (ntiles == 0) {  // an empty split (more splits than context tiles): contributes nothing
+    if (row_ok && a.S > 1 && half == 0) {
+      const int64_t nrows = (int64_t)a.bs * a.H * KL;
+      a.ws_lse[(int64_t)s * nrows + ((int64_t)b * a.H + head) * KL + qi] = -INFINITY;
+    }
+    return;
+  }
   const int last = ntiles - 1;
 
   // ---- direct-to-LDS tile loads. Instruction i (0 .. LPW - 1) of wave w fills the 16-byte chunk positions
@@ -766,7 +686,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))
   // loads live across the tile loops
   int token_e = token, qi_e = qi;
   asm volatile("" : "+v"(token_e), "+v"(qi_e));
-  if (whole) {
+  if (a.S == 1) {
     if (!row_ok) return;
     uint16_t* op = a.out + (int64_t)token_e * a.o_st + (int64_t)head * a.o_sh;
 #pragma unroll
@@ -818,27 +738,20 @@ __global__ __launch_bounds__(256) void mode_attn_merge_kernel(AttnArgs a) {
   const int KL = a.K * a.L;
   const int64_t nrows = (int64_t)a.bs * a.H * KL;
   const int64_t prow = (int64_t)blockIdx.x * 16 + (threadIdx.x >> 4);
-  const int fair = a.fold ? fair_chunk(a) : 0;  // by whole waves
   if (prow >= nrows) return;
   const int d0 = (threadIdx.x & 15) * 8;
-  // partials of this row's request: its context splits that hold keys, then (one request) the block partial SC
-  const int ctx = a.ctx_lens ? (int)a.ctx_lens[prow / ((int64_t)a.H * KL)] : a.ctx_const;
-  const int chunk = split_chunk(a, ctx, fair);
-  const int ns = (ctx + chunk - 1) / chunk;
-  const int np = a.fold ? ns : ns + 1;
-  if (a.fold && np <= 1) return;  // written by its only workgroup
   float m = -INFINITY, tot = 0.f;
   f32x4 acc0 = {0.f, 0.f, 0.f, 0.f}, acc1 = acc0;
-  for (int s0 = 0; s0 < np; s0 += SB) {
+  for (int s0 = 0; s0 < a.S; s0 += SB) {
     float l[SB], ex[SB];
     u32x4 oh[SB];
 #pragma unroll
     for (int j = 0; j < SB; ++j) {
+      const int s = s0 + j;
       l[j] = -INFINITY;
       ex[j] = 0.f;
       oh[j] = (u32x4){0u, 0u, 0u, 0u};
-      if (s0 + j < np) {
-        const int s = !a.fold && s0 + j == ns ? a.SC : s0 + j;
+      if (s < a.S) {  // uniform
         l[j] = a.ws_lse[s * nrows + prow];
         ex[j] = a.ws_exp[s * nrows + prow];
         oh[j] = *reinterpret_cast<const u32x4*>(a.ws_o + (s * nrows + prow) * D + d0);
@@ -856,7 +769,7 @@ __global__ __launch_bounds__(256) void mode_attn_merge_kernel(AttnArgs a) {
     m = mn;
 #pragma unroll
     for (int j = 0; j < SB; ++j)
-      if (l[j] != -INFINITY) {
+      if (l[j] != -INFINITY) {  // an empty split wrote no partial output
         const float wgt = exp2f(l[j] - m);
         const float wo = __builtin_ldexpf(wgt, (int)ex[j]);
         const f32x2 o01 = h2_to_f2(oh[j][0]), o23 = h2_to_f2(oh[j][1]);
@@ -931,8 +844,7 @@ extern "C" int mfd_mode_attn(const uint16_t* q, int64_t q_st, int64_t q_sh, cons
   a.req_idx = req_idx; a.ctx_lens = ctx_lens; a.ctx_const = ctx_len_const;
   a.out = out; a.o_st = o_st; a.o_sh = o_sh;
   const int64_t rows = (int64_t)bs * H * KL;
-  a.fold = num_ctx_splits > 1 && ctx_lens && slot_table && bs > 1;  // (flat contexts keep their even splits)
-  const int SP = num_ctx_splits > 1 ? num_ctx_splits + (a.fold ? 0 : 1) : 1;
+  const int SP = num_ctx_splits > 1 ? num_ctx_splits + 1 : 1;
   a.ws_o = reinterpret_cast<uint16_t*>(workspace);
   a.ws_lse = workspace ? reinterpret_cast<float*>(a.ws_o + (int64_t)SP * rows * D) : nullptr;
   a.ws_exp = workspace ? a.ws_lse + (int64_t)SP * rows : nullptr;
@@ -945,8 +857,6 @@ extern "C" int mfd_mode_attn(const uint16_t* q, int64_t q_st, int64_t q_sh, cons
   // units of a KV head come in eights; four-wave ones (two per CU) otherwise
   const int NW = (units % 8 == 0) ? 8 : NWAVES;
   a.ngroups = (units + NW - 1) / NW;
-  a.per_cu = NW == 8 ? 1 : 2;
-  a.slots = a.per_cu * mfd_num_cus();
   const int P = bs * Hkv * SP;
   const int P8 = (P + 7) / 8;
   hipStream_t st = static_cast<hipStream_t>(stream);

@@ -24,17 +24,15 @@ import mode_attention
 
 
 def resolve_ctx_splits(num_ctx_splits: int, *, programs: int, device) -> int:
-    """num_ctx_splits > 0: at most that many context splits per request (merged by log-sum-exp); 0: one fused pass;
-    < 0: auto. ``programs``: (request, KV head, group of four 32-query units) units of work, of which the chip holds
-    two per CU. One pass once they fill it; else up to four slot counts' worth of splits, between 4 and 16: the kernel,
-    which sees the lengths, splits only the requests that are longer than their share (a batch of 5 requests of 389 to
-    6719 tokens and 160 programs: 140 us with 2 even splits, 60 us so). (P:886-894.)"""
+    """num_ctx_splits > 0: that many context splits (merged by log-sum-exp); 0: one fused pass; < 0: auto —
+    fused once the (request, KV head, unit group) programs cover the CUs, else enough splits to cover them
+    (at most 16). (P:886-894.)"""
     if num_ctx_splits >= 0:
         return num_ctx_splits
-    slots = 2 * mfd_hip.cu_count(device)
-    if programs > slots:
+    want = mfd_hip.cu_count(device)
+    if programs >= want:
         return 0
-    return min(16, max(4, -(-2 * slots // programs) + 2))
+    return min(16, max(1, -(-want // programs)))
 
 
 def paged_mode_block_attention(

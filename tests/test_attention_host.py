@@ -79,3 +79,16 @@ def test_paged_reference_and_hook(page_size):
     with pytest.raises(ValueError):
         dm.PagedModeAttention(kv_pool=Pool(), req_to_token=table, num_modes=8, block_size=16, num_heads=16,
                               num_kv_heads=4, head_dim=128, scaling=1.0, num_ctx_splits=0, impl="cuda")
+
+
+@pytest.mark.parametrize("programs,splits", [(1, 16), (16, 16), (17, 16), (32, 8), (64, 4), (160, 2), (255, 2), (256, 0),
+                                             (416, 0), (2000, 0)])
+def test_auto_ctx_splits(programs, splits, monkeypatch):
+    """Automatic context splits of the paged form on 256 CUs (P:886-894): enough to give every CU a program, at most 16,
+    one pass from a program per CU on; a given count stays as it is."""
+    import mfd_hip
+    import paged_mode_attention as dm
+
+    monkeypatch.setattr(mfd_hip, "cu_count", lambda device: 256)
+    assert dm.resolve_ctx_splits(-1, programs=programs, device="cuda") == splits
+    assert [dm.resolve_ctx_splits(n, programs=programs, device="cuda") for n in (0, 1, 7)] == [0, 1, 7]

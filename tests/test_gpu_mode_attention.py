@@ -91,14 +91,14 @@ def test_paged_per_token_table(lens, splits):
 
 
 @pytest.mark.parametrize("lens,H,Hkv,K,splits,page_size", [
-    ([0, 5, 3000, 64, 129], 16, 8, 8, -1, 64),           # split, whole and empty requests side by side
-    ([700] + [30] * 70, 8, 2, 2, -1, 1),                 # more than 64 requests, one of them split
+    ([0, 5, 3000, 64, 129], 16, 8, 8, -1, 64),           # long, short and empty requests side by side
+    ([700] + [30] * 70, 8, 2, 2, -1, 1),                 # more than 64 requests, one of them long
     ([3000] + list(range(1, 71)), 8, 8, 2, 5, 64),       # more workgroups than the chip holds: longest first
     ([0, 0, 0], 8, 4, 3, 4, 1), ([128, 129, 127], 8, 4, 8, 16, 64), ([4097, 1], 32, 4, 1, -1, 16),
 ])
 def test_paged_split_batches(lens, H, Hkv, K, splits, page_size):
-    """Batches whose requests take as many splits as their lengths ask for: every split count from one (which writes
-    the output itself) to the limit, no request left out and none read past its end."""
+    """Batches of very different lengths under one split count: requests shorter than a split (empty partials), no
+    request left out and none read past its end."""
     d = paged_attention_inputs(90 + len(lens), lens, K=K, H=H, Hkv=Hkv, page_size=page_size)
     table = torch.zeros(len(lens) + 2, d["page_table"].shape[1], dtype=torch.int32)
     table[2:] = d["page_table"]
@@ -106,6 +106,35 @@ def test_paged_split_batches(lens, H, Hkv, K, splits, page_size):
     got = _paged(d, page_size, splits, d["req_to_token"] if page_size == 1 else table)
     torch.cuda.synchronize()
     _check(got, _paged_ref(d), f"split batch {lens[:6]}")
+
+
+@pytest.mark.parametrize("page_size", [1, 64])
+def test_paged_split_request_independent_of_batch(page_size):
+    """With a split count given, a request's output has the same bits whatever else is in the batch: its splits follow
+    from its own length alone."""
+    lens = [3000, 64, 700, 0, 129]
+    d = paged_attention_inputs(7, lens, K=4, H=16, Hkv=4, page_size=page_size)
+    table = torch.zeros(len(lens) + 2, d["page_table"].shape[1], dtype=torch.int32)
+    table[2:] = d["page_table"]
+    table = d["req_to_token"] if page_size == 1 else table
+    print(f"case: split request alone and in a batch, page_size={page_size}", flush=True)
+    got = _paged(d, page_size, 3, table).cpu()
+    KL = d["num_modes"] * d["block_size"]
+    for b in range(len(lens)):
+        rows = slice(b * KL, (b + 1) * KL)
+        one = dict(d, q=d["q"][rows], k_new=d["k_new"][rows], v_new=d["v_new"][rows], ctx_lens=d["ctx_lens"][b:b + 1],
+                   req_pool_indices=d["req_pool_indices"][b:b + 1])
+        assert torch.equal(_paged(one, page_size, 3, table).cpu(), got[rows]), b
+
+
+def test_paged_auto_splits_one_pass_from_a_program_per_cu():
+    """Eight requests of 32 / 8 heads, 8 modes x 16: 256 (request, KV head, unit group) programs, a workgroup for every
+    CU. The automatic choice is one pass then, bit for bit: O stays in fp32 up to the output, no fp16 partials."""
+    d = paged_attention_inputs(8, [3000, 40, 129, 64, 500, 1, 900, 77], K=8, H=32, Hkv=8, page_size=1)
+    print("case: automatic splits at 256 programs", flush=True)
+    auto, whole = _paged(d, 1, -1, d["req_to_token"]), _paged(d, 1, 0, d["req_to_token"])
+    torch.cuda.synchronize()
+    assert torch.equal(auto, whole)
 
 
 def test_paged_64_token_pages_config4_heads():
