@@ -351,6 +351,11 @@ __device__ float row_logz(const TopkArgs& a, int row, const PieceSums& p, double
 constexpr int NBIN = 1024;
 constexpr int COUNT_MAX = 256;  // up to here a candidate's rank is counted against all others
 constexpr int CAND_MAX = 1024;
+// Counters of the bisections: one for each of the 16 bits of a key, one for the elements above it, one for each bit of
+// an element's index (k = 1 takes MERGE_MAX pieces: up to 2^24 elements, whose number has 25 bits)
+constexpr int VBITS = 32 - __builtin_clz(MERGE_MAX * PIECE);
+constexpr int NCOUNT = 16 + 1 + VBITS;
+static_assert((int64_t)MERGE_MAX * PIECE < (int64_t)1 << 31 && NCOUNT <= 64, "cleared by one wave");
 struct MergeLds {
   uint32_t hist[NBIN];
   __attribute__((aligned(16))) uint64_t cand[CAND_MAX + 2];
@@ -358,7 +363,7 @@ struct MergeLds {
   uint16_t bnd[CAND_MAX];
   uint16_t glist[2 * KMAX];  // the groups whose elements are looked at
   int wsum[16];
-  int count[40];
+  int count[NCOUNT];
   int n, nsel, nb, bin, need, ng, top;
   float logz;
 };
@@ -525,7 +530,7 @@ __device__ void row_topk(const TopkArgs& a, int row, MergeLds& ml, double* terms
     ml.n = 0;
     ml.bin = -1;
   }
-  if (tid < 40) ml.count[tid] = 0;
+  if (tid < NCOUNT) ml.count[tid] = 0;
   int top = KEY_MIN;
   for_groups([&](int key, int) { top = std::max(top, key); });
   top = wave_max_i32(top);
@@ -556,7 +561,7 @@ __device__ void row_topk(const TopkArgs& a, int row, MergeLds& ml, double* terms
     }
     t = (int)T - 32768;
     __syncthreads();
-    if (tid < 40) ml.count[tid] = 0;
+    if (tid < NCOUNT) ml.count[tid] = 0;
   }
   if (t == 0) t = -1;  // -0 counts as 0
   auto at_t = [&](int key) -> bool { return t == -1 ? key == 0 || key == -1 : key == t; };

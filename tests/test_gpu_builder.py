@@ -96,6 +96,27 @@ def test_topk_logz_selection_edges(kind, rows, V, k):
     np.testing.assert_array_equal(logp.cpu().numpy().view(np.uint32), lp_ref.view(np.uint32))
 
 
+@pytest.mark.parametrize("V,k,first", [(1 << 22, 2, 5), (1 << 23, 2, 0), (1 << 23, 2, 4194311), ((1 << 23) - 8, 2, 8),
+                                       (1 << 23, 1, 8388001), (1 << 24, 1, 0), (1 << 24, 1, 8388619)])
+def test_topk_logz_ties_of_the_longest_rows(V, k, first):
+    """Rows up to the longest accepted for k = 1 and 2, equal values from one column on: their first columns are found by
+    bisection over every bit of a column number. log Z to fp32 rounding of the exact value."""
+    import tree_logits
+
+    x = torch.full((2, V), -5.0, dtype=torch.bfloat16, device="cuda")
+    x[0, first:] = 1.5
+    x[1, :first] = 1.5  # (first = 0: all equal)
+    print(f"case: topk_logz ties V={V} k={k} first={first}", flush=True)
+    logp, ids, logz = tree_logits.topk_logz(x, k, with_logz=True)
+    torch.cuda.synchronize()
+    assert ids.tolist() == [[first + j for j in range(k)], list(range(k))]
+    for r, n in enumerate((V - first, first)):
+        top = 1.5 if n else -5.0
+        ref = top + np.log(n + (V - n) * np.exp(-6.5)) if n else top + np.log(V)
+        assert abs(logz[r].item() - ref) <= 2e-6 * abs(ref)
+        np.testing.assert_allclose(logp[r].cpu().numpy(), top - ref, rtol=2e-6)
+
+
 def test_row_logsumexp_and_top_candidates_api():
     import tree_logits
 
