@@ -28,11 +28,18 @@ class ModeBlocks:
         self.exact = exact  # checks only: float32 reference() instead of the kernel
 
 
+def unit_groups(group: int, num_queries: int) -> int:
+    """Groups of four units of one KV head, as the kernel forms them: a unit is 32 queries of one of the KV head's
+    ``group`` query heads, a head's last unit padded."""
+    return -(-(group * -(-num_queries // 32)) // 4)
+
+
 def _auto_splits(programs: int, ctx: int, device) -> int:
     """Context splits for num_ctx_splits < 0: the most for which the whole grid (per program the context splits
     plus the block partial) fits one round of workgroup slots, two per CU, keeping >= 256 keys per split; one
     pass when no second split fits. (A grid one slot round larger runs a second round: config 2 measures 29.4-29.8
-    us with 13-15 splits, 31 us with 12, 37 us with 16.)"""
+    us with 13-15 splits, 31 us with 12, 37 us with 16. 40 heads over 8, 3 modes x 16: 24 programs, 20 splits and 31 us
+    at 8000 keys, 40 us with the 31 splits that a count of 16 programs, without the padding of each head, allows.)"""
     if ctx <= 256:
         return 1
     slots = 2 * mfd_hip.cu_count(device)
@@ -70,7 +77,7 @@ def mode_block_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, num_
     mfd_hip.require_cuda(q, k, v)
     ctx = total - num_queries
     G = num_heads // num_kv_heads
-    programs = num_kv_heads * -(-(G * num_queries // 32) // 4)
+    programs = num_kv_heads * unit_groups(G, num_queries)
     if num_ctx_splits < 0:
         splits = _auto_splits(programs, ctx, q.device)
     else:

@@ -35,6 +35,12 @@ def resolve_ctx_splits(num_ctx_splits: int, *, programs: int, device) -> int:
     return min(16, max(1, -(-want // programs)))
 
 
+def _programs(bs: int, num_kv_heads: int, group: int, num_queries: int) -> int:
+    """(request, KV head, group of 128 query rows) programs of a batch: the rows of a KV head's query heads together,
+    whole 32-row units of them, at least one."""
+    return bs * num_kv_heads * max(1, -(-(group * num_queries // 32) // 4))
+
+
 def paged_mode_block_attention(
     *,
     q: torch.Tensor,
@@ -77,8 +83,7 @@ def paged_mode_block_attention(
     if bs == 0:
         return out
     G = H // Hkv
-    programs = bs * Hkv * -(-(G * KL // 32) // 4)
-    splits = resolve_ctx_splits(num_ctx_splits, programs=programs, device=q.device)
+    splits = resolve_ctx_splits(num_ctx_splits, programs=_programs(bs, Hkv, G, KL), device=q.device)
     rpi = req_pool_indices[:bs]
     if rpi.dtype != torch.int64:
         rpi = rpi.to(torch.int64)

@@ -92,3 +92,27 @@ def test_auto_ctx_splits(programs, splits, monkeypatch):
     monkeypatch.setattr(mfd_hip, "cu_count", lambda device: 256)
     assert dm.resolve_ctx_splits(-1, programs=programs, device="cuda") == splits
     assert [dm.resolve_ctx_splits(n, programs=programs, device="cuda") for n in (0, 1, 7)] == [0, 1, 7]
+
+
+@pytest.mark.parametrize("H,Hkv", [(8, 8), (16, 8), (32, 8), (40, 8), (32, 4)])
+@pytest.mark.parametrize("KL", [1, 7, 8, 14, 16, 48, 128])
+def test_auto_ctx_splits_of_small_and_padded_blocks(H, Hkv, KL, monkeypatch):
+    """Fewer than 32 query rows per KV head, and heads whose last 32-query unit is padded: the flat form's grid (the
+    context splits and the block partial of every workgroup of the kernel) fits one round of the chip's slots, the paged
+    form counts at least one program per request and KV head."""
+    import mfd_hip
+    import mode_attention
+    import paged_mode_attention as dm
+
+    monkeypatch.setattr(mfd_hip, "cu_count", lambda device: 256)
+    G = H // Hkv
+    units = G * ((KL + 31) // 32)
+    nw = 8 if units % 8 == 0 else 4  # the kernel's waves per workgroup: one workgroup of eight per CU, two of four
+    wgs, slots = Hkv * ((units + nw - 1) // nw), 256 if nw == 8 else 512
+    for ctx in (257, 2000, 8000, 32768):
+        splits = mode_attention._auto_splits(Hkv * mode_attention.unit_groups(G, KL), ctx, "cuda")
+        assert splits >= 2 and wgs * (splits + 1) <= slots and splits <= -(-ctx // 256)
+    for bs in (1, 3):
+        programs = dm._programs(bs, Hkv, G, KL)
+        assert programs >= bs * Hkv
+        assert 1 <= dm.resolve_ctx_splits(-1, programs=programs, device="cuda") <= 16

@@ -137,6 +137,20 @@ def test_paged_auto_splits_one_pass_from_a_program_per_cu():
     assert torch.equal(auto, whole)
 
 
+@pytest.mark.parametrize("K,bs,H,Hkv", [(1, 7, 16, 8), (1, 7, 32, 8), (1, 1, 8, 8), (2, 7, 16, 8), (3, 16, 40, 8)])
+def test_auto_splits_of_small_blocks(K, bs, H, Hkv):
+    """Automatic splits with fewer than 32 query rows per KV head, and with a padded last unit in every head."""
+    import mode_attention
+
+    print(f"case: auto splits K={K} bs={bs} H={H}/{Hkv}", flush=True)
+    q, k, v = attention_inputs(K * bs, K=K, bs=bs, H=H, Hkv=Hkv, ctx=700)
+    got = mode_attention.mode_block_attention(q.cuda(), k.cuda(), v.cuda(), K, bs, 128 ** -0.5, num_ctx_splits=-1)
+    ref = att.mode_attention(q.float().numpy(), k.float().numpy(), v.float().numpy(), K, bs, 128 ** -0.5)
+    _check(got, ref, f"flat {K}x{bs}")
+    d = paged_attention_inputs(K * bs, [700, 40], K=K, bs=bs, H=H, Hkv=Hkv, page_size=1)
+    _check(_paged(d, 1, -1, d["req_to_token"]), _paged_ref(d), f"paged {K}x{bs}")
+
+
 def test_paged_64_token_pages_config4_heads():
     """Config 4 attention shapes (40 q heads over 8 KV heads, K=8 x 16), 64-token pages, U[1024, 8192] contexts."""
     g = torch.Generator().manual_seed(4000)
