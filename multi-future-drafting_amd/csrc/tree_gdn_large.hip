@@ -879,11 +879,12 @@ int run_large(const GdnLargeArgs& a, int max_nodes, hipStream_t s) {
   }
   if (b.gsync)
     return wide ? run_large_ct<NMAX, 2, true, false>(b, nml, s) : run_large_ct<NMAX, 1, true, false>(b, nml, s);
-  if (NMAX <= TWO_NODES || nml <= TWO_NODES)
+  // two workgroups per CU only where a CU has a second one to overlap with. In a grid of one round (four layers with
+  // their context) the form costs more than it gives: 2 x 257 nodes, HK 16 / H 32, 117 us against 105 with one; 1 x 257,
+  // 16 / 16, 88 against 83; 4 x 200, 16 / 16, 102 against 90
+  if ((int64_t)8 * P8 * SUB > cus && nml <= TWO_NODES)
     return wide ? run_large_ct<NMAX, 2, false, true>(b, nml, s) : run_large_ct<NMAX, 1, false, true>(b, nml, s);
-  if constexpr (NMAX > TWO_NODES)
-    return wide ? run_large_ct<NMAX, 2, false, false>(b, nml, s) : run_large_ct<NMAX, 1, false, false>(b, nml, s);
-  return MFD_OK;
+  return wide ? run_large_ct<NMAX, 2, false, false>(b, nml, s) : run_large_ct<NMAX, 1, false, false>(b, nml, s);
 }
 
 }  // namespace

@@ -100,6 +100,24 @@ def test_tree_gdn_large_two_per_cu(sizes, HK, H):
     _check(u, o, d, f"{sizes}")
 
 
+@pytest.mark.parametrize("sizes,HK,H", [
+    ([257, 130], 16, 32),             # 256 workgroups of 32 columns, more chunks than workgroups of a group
+    ([272], 16, 16),                  # the same with 16 columns
+    ([200, 129, 256, 3], 16, 16),     # the 256-node layout
+    ([144, 130, 200, 9, 40], 16, 16), # one request more: two workgroups per CU
+])
+def test_tree_gdn_large_grids_of_one_round(sizes, HK, H):
+    """Grids of at most one workgroup per CU (256) that the one-launch form does not take."""
+    import tree_gdn_kernel
+
+    d = gdn_inputs(sizes, HK, H, 128, seed=sum(sizes) + H + 1)
+    t = _dev(d)
+    print(f"case: one round {sizes} HK={HK} H={H}", flush=True)
+    u, o = tree_gdn_kernel.tree_gdn_varlen(t["q"], t["k"], t["v"], t["g_cum"], t["beta"], t["s0"], t["parents"],
+                                           t["cu_nodes"], max_nodes=max(sizes))
+    _check(u, o, d, f"{sizes}")
+
+
 def test_tree_gdn_large_one_launch_two_streams():
     """Two streams running the one-launch form at once (one 257-node tree each, HK 16 / H 32: 256 workgroups per
     call, so the second call's workgroups start as the first's end): each stream has hand-over words of its own."""
