@@ -4,8 +4,8 @@
 // g = -exp(float(A_log)) * softplus(float(a) + float(dt_bias)) (torch's softplus: x above 20 is returned
 // as is, else log1p(exp(x))), and G = anc @ g, the log decay summed over the node's ancestors and itself.
 // The reference forms G with a dense [n, n] x [n, H] product; here a workgroup takes one request's nodes with four
-// heads: g of every (node, head) and every node's root path (parents precede children, so the walk up the parent
-// pointers ends at the root) go to LDS, then each (node, head) thread sums g over the path from the root down.
+// heads: the softplus of every (node, head) and every node's root path (parents precede children, so the walk up the
+// parent pointers ends at the root) go to LDS, then each (node, head) thread sums g over the path from the root down.
 #include "mfd_common.h"
 
 namespace {
@@ -35,16 +35,16 @@ __device__ __forceinline__ float load_ab(const void* p, int ab_bf16, int64_t idx
 __device__ __forceinline__ float softplus_torch(float x) { return x > 20.f ? x : log1pf(expf(x)); }
 
 // What bounds it: latency, that of two trips to memory (offsets, then parents and projections) and of the chain of a
-// few hundred dependent operations of softplus and sigmoid, which a CU with one wave per SIMD cannot hide: so g is
-// formed once per (node, head), by all threads at once. 8 trees of 128 nodes, 32 heads: 5.5 us; 11 us with g formed
-// again for every descendant, 16.8 us for threads that walked in memory, once per summed ancestor.
+// few hundred dependent operations of softplus and sigmoid, which the two waves per SIMD of a CU's one workgroup do not
+// hide: so the softplus is formed once per (node, head), by all threads at once. 8 trees of 128 nodes, 32 heads: 5.5 us;
+// 11 us with g formed again for every descendant, 16.8 us for threads that walked in memory, once per summed ancestor.
 constexpr int NT = 512;
 constexpr int HB = 4;       // heads per workgroup: 64 workgroups for 8 requests of 32 heads
 constexpr int NMAX = 1024;  // nodes of a request held in LDS; a larger request's threads walk in memory
 constexpr int PATH = 16;    // path entries held in LDS; deeper nodes walk again per ancestor
 
 __global__ __launch_bounds__(NT) void tree_gates_kernel(GatesArgs a) {
-  __shared__ float g[NMAX][HB];
+  __shared__ float sp[NMAX][HB];  // softplus of every (node, head)
   __shared__ int16_t par[NMAX];
   __shared__ uint16_t path[NMAX][PATH];  // [s] = the s-th ancestor (0 = the node itself), request-local
   const int tid = threadIdx.x;
@@ -55,9 +55,9 @@ __global__ __launch_bounds__(NT) void tree_gates_kernel(GatesArgs a) {
   const int n = (a.cu_nodes && r + 1 < a.R ? a.cu_nodes[r + 1] : a.N) - ns;  // the last request ends the batch
   const bool live = h < a.H;
   const float dt = live ? a.dt_bias[h] : 0.f, scale = live ? -expf(a.A_log[h]) : 0.f;
-  auto g_at = [&](int i) -> float {
-    const float x = load_ab(a.a, a.ab_bf16, (int64_t)(ns + i) * a.ab_st + h) + dt;
-    return scale * softplus_torch(x);
+  // (the sum over a path takes each g = scale * softplus as the product of an FMA, rounded once with the sum)
+  auto softplus_at = [&](int i) -> float {
+    return softplus_torch(load_ab(a.a, a.ab_bf16, (int64_t)(ns + i) * a.ab_st + h) + dt);
   };
   // parent of a request-local node in memory: from the parents, or the largest strict ancestor in anc8
   auto parent_of = [&](int i) -> int {
@@ -105,7 +105,7 @@ __global__ __launch_bounds__(NT) void tree_gates_kernel(GatesArgs a) {
     if (live) {
       const int64_t at = (int64_t)(ns + i) * a.H + h;
       a.beta[at] = 1.f / (1.f + expf(-load_ab(a.b, a.ab_bf16, (int64_t)(ns + i) * a.ab_st + h)));
-      if (staged) g[i][tid & (HB - 1)] = g_at(i);
+      if (staged) sp[i][tid & (HB - 1)] = softplus_at(i);
     }
   }
   __syncthreads();
@@ -135,16 +135,22 @@ __global__ __launch_bounds__(NT) void tree_gates_kernel(GatesArgs a) {
       if (a.err) atomicOr(a.err, MFD_DEVERR_NOT_TOPOLOGICAL);
       G = __builtin_nanf("");
     } else if (staged && d <= PATH) {
+      // all reads in flight before the first sum, each pinned outside its select (left free, the compiler puts every
+      // read and sum behind a branch of its own)
+      float x[PATH];
+#pragma unroll
+      for (int s = PATH - 1; s >= 0; --s) x[s] = sp[path[i][s < d ? s : 0]][tid & (HB - 1)];
 #pragma unroll
       for (int s = PATH - 1; s >= 0; --s) {
-        const float x = g[path[i][s < d ? s : 0]][tid & (HB - 1)];
-        G = s < d ? G + x : G;
+        asm volatile("" : "+v"(x[s]));
+        const float with = fmaf(scale, x[s], G);
+        G = s < d ? with : G;
       }
     } else {
       for (int s = d - 1; s >= 0; --s) {  // s = steps from the node up to the summed ancestor
         int cur = i;
         for (int q = 0; q < s; ++q) cur = up(cur);
-        G += staged ? g[cur][tid & (HB - 1)] : g_at(cur);
+        G = fmaf(scale, staged ? sp[cur][tid & (HB - 1)] : softplus_at(cur), G);
       }
     }
     a.g_cum[(int64_t)(ns + i) * a.H + h] = G;

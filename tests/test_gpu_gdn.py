@@ -378,6 +378,47 @@ def test_tree_gates_deep_long_and_many_requests(case):
     np.testing.assert_allclose(G.cpu().numpy(), G_ref, rtol=0, atol=1e-5 * np.abs(G_ref).max())
 
 
+def _round_f32(x):
+    """A Fraction rounded to float32, to nearest (even on ties)."""
+    from fractions import Fraction
+
+    c = np.float32(float(x))
+    near = [np.nextafter(c, np.float32(-np.inf)), c, np.nextafter(c, np.float32(np.inf))]
+    return min(near, key=lambda y: (abs(Fraction(float(y)) - x), int(y.view(np.uint32)) & 1))
+
+
+@pytest.mark.parametrize("n,depth", [(60, 12), (40, 40), (1100, 30)])
+def test_tree_gates_one_rounding_per_ancestor(n, depth):
+    """G takes each ancestor's -exp(A_log) * softplus by an FMA: product and sum are rounded once. Above 20 softplus(x)
+    is x, and a root with x = 32 shows the kernel's own exp(A_log), so the sums are known to the last bit. Paths short
+    and long, requests in and beyond the workgroup's LDS."""
+    import tree_gdn_kernel
+    from fractions import Fraction
+
+    rng = np.random.default_rng(n)
+    H = 6
+    parents = np.array([i - 1 if i < depth else rng.integers(0, min(i, depth)) for i in range(n)], dtype=np.int32)
+    x = rng.uniform(21, 60, (n, H)).astype(np.float32)
+    x[0] = 32
+    A_log = rng.standard_normal(H).astype(np.float32)
+    dev = lambda t: torch.from_numpy(t).cuda()
+    print(f"case: gates roundings n={n} depth={depth}", flush=True)
+    G, _ = tree_gdn_kernel.tree_gates(dev(x), dev(x), dev(A_log), torch.zeros(H, device="cuda"), parents=dev(parents))
+    G = G.cpu().numpy()
+    scale = G[0] / np.float32(32)  # exact
+    np.testing.assert_allclose(scale, -np.exp(A_log), rtol=1e-6)
+    nodes = np.concatenate([np.arange(min(n, depth)), rng.choice(n, min(n, 80), replace=False)])
+    for i in nodes:
+        path = [int(i)]
+        while parents[path[-1]] >= 0:
+            path.append(int(parents[path[-1]]))
+        for h in range(H):
+            g = np.float32(0)
+            for j in reversed(path):
+                g = _round_f32(Fraction(float(scale[h])) * Fraction(float(x[j, h])) + Fraction(float(g)))
+            assert g == G[i, h], (i, h)
+
+
 def test_tree_gates_anc8_and_into_tree_gdn():
     """Single tree given by its ancestor matrix (the HF TreeContext form); the gates then feed tree_gdn,
     which must match the oracle fed with the oracle's gates."""
