@@ -419,6 +419,31 @@ def test_tree_gates_one_rounding_per_ancestor(n, depth):
             assert g == G[i, h], (i, h)
 
 
+@pytest.mark.parametrize("n,first", [(293, 5), (1403, 8)])
+def test_tree_gates_anc8_far_parents(n, first):
+    """A tree given by its ancestor matrix, rows of odd length, parents more than 256 entries before their children;
+    1403 nodes are beyond the workgroup's LDS."""
+    import tree_gdn_kernel
+
+    rng = np.random.default_rng(n)
+    H = 5
+    parents = np.array([min(i - 1, int(rng.integers(0, first))) if i else -1 for i in range(n)], dtype=np.int32)
+    g = torch.Generator().manual_seed(n)
+    a, b = torch.randn(n, H, generator=g), torch.randn(n, H, generator=g)
+    A_log, dt = torch.randn(H, generator=g) * 0.5, torch.randn(H, generator=g)
+    anc8 = torch.from_numpy(gdn.ancestor_matrix(parents).astype(np.int8)).cuda()
+    print(f"case: gates anc8 n={n}", flush=True)
+    G, beta = tree_gdn_kernel.tree_gates(a.cuda(), b.cuda(), A_log.cuda(), dt.cuda(), anc8=anc8)
+    same, same_beta = tree_gdn_kernel.tree_gates(a.cuda(), b.cuda(), A_log.cuda(), dt.cuda(),
+                                                 parents=torch.from_numpy(parents).cuda())
+    torch.cuda.synchronize()
+    G_ref, beta_ref = _gates_ref(a, b, A_log, dt, parents, [0, n], torch.float32)
+    np.testing.assert_allclose(beta.cpu().numpy(), beta_ref, rtol=0, atol=1e-6)
+    # fp32 sums of at most first + 1 terms of one sign
+    np.testing.assert_allclose(G.cpu().numpy(), G_ref, rtol=0, atol=1e-5 * np.abs(G_ref).max())
+    assert torch.equal(G, same) and torch.equal(beta, same_beta)
+
+
 def test_tree_gates_anc8_and_into_tree_gdn():
     """Single tree given by its ancestor matrix (the HF TreeContext form); the gates then feed tree_gdn,
     which must match the oracle fed with the oracle's gates."""
