@@ -351,6 +351,7 @@ __device__ float row_logz(const TopkArgs& a, int row, const PieceSums& p, double
 constexpr int NBIN = 1024;
 constexpr int COUNT_MAX = 256;  // up to here a candidate's rank is counted against all others
 constexpr int CAND_MAX = 1024;
+constexpr int TIED_MAX = 512;   // k <= 32: beyond, the bisection
 // Counters of the bisections: one for each of the 16 bits of a key, one for the elements above it, one for each bit of
 // an element's index (k = 1 takes MERGE_MAX pieces: up to 2^24 elements, whose number has 25 bits)
 constexpr int VBITS = 32 - __builtin_clz(MERGE_MAX * PIECE);
@@ -362,7 +363,7 @@ struct MergeLds {
   __attribute__((aligned(16))) uint64_t sel[KMAX];
   uint16_t bnd[CAND_MAX];
   uint16_t glist[2 * KMAX];  // the groups whose elements are looked at
-  int wsum[16];
+  int wmax[16], wsum[16];
   int count[NCOUNT];
   int n, nsel, nb, bin, need, ng, top;
   float logz;
@@ -418,14 +419,13 @@ __device__ __forceinline__ bool kth_bin(const uint32_t* hist, int k, int* bin, i
 // counting, n broadcast reads each. More: the value keys' distance from the largest, clamped to 1024 bins, is
 // histogrammed, the bin that holds the k-th largest is read off the suffix sums, the candidates above it are taken,
 // those in it by their rank among themselves (one value unless clamped, so ties by token id), and the k taken are
-// ranked by counting, four threads each.
+// ranked by counting, four threads each. False, with nothing written, if that bin holds more than max_tied candidates.
 template <int NTH>
-__device__ void merge_row(const TopkArgs& a, int row, int n, int top, MergeLds& ml) {
+__device__ bool merge_row(const TopkArgs& a, int row, int n, int top, int max_tied, MergeLds& ml) {
   const int tid = threadIdx.x;
   const int k = a.k;
   uint64_t* cand = ml.cand;
   const float logz = ml.logz;
-  if (tid == 0 && a.out_logz) a.out_logz[row] = logz;
   if (n <= COUNT_MAX) {
     if (tid < n) {
       const uint64_t v = cand[tid];
@@ -436,7 +436,7 @@ __device__ void merge_row(const TopkArgs& a, int row, int n, int top, MergeLds& 
       }
       if (r < k) put_one(a, row, r, v, logz);
     }
-    return;
+    return true;
   }
   for (int i = tid; i < NBIN; i += NTH) ml.hist[i] = 0;
   if (tid < KMAX) ml.sel[tid] = 0;
@@ -451,6 +451,7 @@ __device__ void merge_row(const TopkArgs& a, int row, int n, int top, MergeLds& 
   if (tid < 64) kth_bin(ml.hist, k, &ml.bin, &ml.need);
   __syncthreads();
   const int bin = ml.bin, need = ml.need;
+  if ((int)ml.hist[bin] > max_tied) return false;
   for (int i = tid; i < n; i += NTH) {
     const uint64_t v = cand[i];
     const int b = bin_of(v);
@@ -481,6 +482,7 @@ __device__ void merge_row(const TopkArgs& a, int row, int n, int top, MergeLds& 
   r += __builtin_amdgcn_update_dpp(0, r, 0xB1, 0xF, 0xF, false);  // lane ^ 1
   r += __builtin_amdgcn_update_dpp(0, r, 0x4E, 0xF, 0xF, false);  // lane ^ 2
   if (s < k && (tid & 3) == 0) put_one(a, row, r, v, logz);
+  return true;
 }
 
 // Kernel 2's work for one row, by all NTH threads of a workgroup, once the row's (m, S) and group keys are in memory.
@@ -534,20 +536,26 @@ __device__ void row_topk(const TopkArgs& a, int row, MergeLds& ml, double* terms
   int top = KEY_MIN;
   for_groups([&](int key, int) { top = std::max(top, key); });
   top = wave_max_i32(top);
-  if (lane == 0) ml.wsum[w] = top;
+  if (lane == 0) ml.wmax[w] = top;
   __syncthreads();
 #pragma unroll
-  for (int i = 0; i < NW; ++i) top = std::max(top, ml.wsum[i]);
-  for_groups([&](int key, int) {
-    const int d = NBIN - 1 - (top - key);
-    if (d >= 0) atomicAdd(&ml.hist[d], 1u);
-  });
-  __syncthreads();
-  if (w == 0) kth_bin(ml.hist, k, &ml.bin, &ml.need);
-  __syncthreads();
-  int t = top - (NBIN - 1 - ml.bin);
-  if (ml.bin < 0) {
-    // further down than the bins reach, or fewer than k groups (then the lowest key)
+  for (int i = 0; i < NW; ++i) top = std::max(top, ml.wmax[i]);
+  const int lsh = a.ng == 16 ? 4 : 6;  // a group is 8 << lsh elements
+  int t = k == 1 ? top : KEY_MIN;      // KEY_MIN: fewer than k groups, every element is taken
+  bool below = false;
+  if (k > 1 && (a.V + (8 << lsh) - 1) >> (lsh + 3) >= k) {
+    for_groups([&](int key, int) {
+      const int d = NBIN - 1 - (top - key);
+      if (d >= 0) atomicAdd(&ml.hist[d], 1u);
+    });
+    __syncthreads();
+    if (w == 0) kth_bin(ml.hist, k, &ml.bin, &ml.need);
+    __syncthreads();
+    below = ml.bin < 0;
+    t = top - (NBIN - 1 - ml.bin);
+  }
+  if (below) {
+    // further down than the bins reach
     uint32_t T = 0;
 #pragma unroll 1
     for (int bit = 15; bit >= 0; --bit) {
@@ -593,7 +601,6 @@ __device__ void row_topk(const TopkArgs& a, int row, MergeLds& ml, double* terms
   __syncthreads();
   // The listed groups' elements, eight per lane and step: step u is 16 or 64 lanes' share of a group.
   const uint16_t* src = a.logits + (int64_t)row * a.row_stride;
-  const int lsh = a.ng == 16 ? 4 : 6;
   const int steps = nl << lsh;
   auto start_of = [&](int u) -> int { return 8 * (((int)ml.glist[u >> lsh] << lsh) + (u & ((1 << lsh) - 1))); };
   if (w == 0) {
@@ -601,7 +608,7 @@ __device__ void row_topk(const TopkArgs& a, int row, MergeLds& ml, double* terms
     if (lane == 0) ml.logz = z;
   } else {
     constexpr int ST = NTH - 64;
-    const i16x2 below = {(int16_t)(t - 1), (int16_t)(t - 1)};  // t > KEY_MIN here or every element is taken
+    const i16x2 under = {(int16_t)(t - 1), (int16_t)(t - 1)};  // t > KEY_MIN here or every element is taken
     for (int u0 = tid - 64 - lane; u0 < steps; u0 += 4 * ST) {
       u32x4 x[4];
       int i0[4];
@@ -619,7 +626,7 @@ __device__ void row_topk(const TopkArgs& a, int row, MergeLds& ml, double* terms
         for (int q = 0; q < 4; ++q) {
           // key > t - 1: the sign of the saturated difference, in both halves
           const uint32_t d = __builtin_bit_cast(
-              uint32_t, __builtin_elementwise_sub_sat(below, __builtin_bit_cast(i16x2, keys2(x[h][q]))));
+              uint32_t, __builtin_elementwise_sub_sat(under, __builtin_bit_cast(i16x2, keys2(x[h][q]))));
           m |= (((d >> 15) & 1u) | ((d >> 30) & 2u)) << (2 * q);
         }
         if (t == KEY_MIN) m = 0xFFu;
@@ -642,10 +649,13 @@ __device__ void row_topk(const TopkArgs& a, int row, MergeLds& ml, double* terms
     }
   }
   __syncthreads();
-  int n = ml.n;
-  // (more than COUNT_MAX candidates for k <= 32 are ties, which the bisection settles sooner than counting them against
-  // each other: a row of 151936 equal values, k = 8, 37 against 86 us)
-  if (n > (k <= 32 ? COUNT_MAX : CAND_MAX)) {
+  const int n = ml.n;
+  if (tid == 0 && a.out_logz) a.out_logz[row] = ml.logz;
+  // (For k <= 32 hundreds of candidates are a row of few groups, or one whose largest values lie close together, or
+  // ties. 8 rows, k = 8, by the bisection and so: 512 values 35 -> 11 us, 20000 falling from the first column on 35 -> 13,
+  // 151936 sorted 39 -> 16. Many equal ones are settled sooner by the bisection than by counting them against each
+  // other: 151936 equal values 41 against 86.)
+  if (n > CAND_MAX || !merge_row<NTH>(a, row, n, top + 32768, k <= 32 ? TIED_MAX : CAND_MAX, ml)) {
     auto norm = [](int key) -> int { return key == -1 ? 0 : key; };
     auto elem = [](const u32x4& x, int e) -> uint16_t { return (uint16_t)((e & 1) ? x[e >> 1] >> 16 : x[e >> 1] & 0xFFFFu); };
     auto for_elements = [&](auto visit) {  // visit(the eight elements, the index of the first)
@@ -694,9 +704,8 @@ __device__ void row_topk(const TopkArgs& a, int row, MergeLds& ml, double* terms
       }
     });
     __syncthreads();
-    n = k;
+    merge_row<NTH>(a, row, k, top + 32768, CAND_MAX, ml);
   }
-  merge_row<NTH>(a, row, n, top + 32768, ml);
 }
 
 // ---- kernel 1 -------------------------------------------------------------------------------------------

@@ -96,6 +96,38 @@ def test_topk_logz_selection_edges(kind, rows, V, k):
     np.testing.assert_array_equal(logp.cpu().numpy().view(np.uint32), lp_ref.view(np.uint32))
 
 
+@pytest.mark.parametrize("kind", ["randn", "front", "sorted", "equal", "ties512", "ties513", "masked_low", "zeros"])
+@pytest.mark.parametrize("V,k", [(300, 8), (511, 1), (900, 8), (1024, 2), (1025, 8), (3000, 24), (4095, 32), (4096, 31),
+                                 (33000, 8), (40001, 3), (40001, 1)])
+def test_topk_logz_close_candidates(kind, V, k):
+    """k <= 32 with more candidates than are counted against each other: rows of fewer than k groups, largest values
+    close together (falling from the first column on, sorted), and ties on both sides of the number that the bisection
+    takes over from."""
+    import tree_logits
+
+    g = torch.Generator().manual_seed(V + k)
+    if kind in ("equal", "masked_low", "zeros"):
+        x = _edge_logits(kind, 3, V, k, V + k)
+    else:
+        x = torch.randn(3, V, generator=g)
+        if kind == "front":
+            x = x + 12 * torch.exp(-torch.arange(V) / 1000.0)
+        elif kind == "sorted":
+            x = torch.sort(x, dim=1).values
+        elif kind.startswith("ties"):
+            at = torch.randperm(min(V, 1024), generator=g)[: int(kind[4:])]
+            x[:, at] = 7.0
+            x[1, at[0]] = 9.0
+        x = x.to(torch.bfloat16)
+    print(f"case: topk_logz close {kind} V={V} k={k}", flush=True)
+    logp, ids, logz = tree_logits.topk_logz(x.cuda(), k, with_logz=True)
+    torch.cuda.synchronize()
+    lp_ref, ids_ref, lz_ref = B.top_candidates(x, k)
+    np.testing.assert_array_equal(ids.cpu().numpy(), ids_ref)
+    np.testing.assert_array_equal(logz.cpu().numpy().view(np.uint32), lz_ref.view(np.uint32))
+    np.testing.assert_array_equal(logp.cpu().numpy().view(np.uint32), lp_ref.view(np.uint32))
+
+
 @pytest.mark.parametrize("V,k,first", [(1 << 22, 2, 5), (1 << 23, 2, 0), (1 << 23, 2, 4194311), ((1 << 23) - 8, 2, 8),
                                        (1 << 23, 1, 8388001), (1 << 24, 1, 0), (1 << 24, 1, 8388619)])
 def test_topk_logz_ties_of_the_longest_rows(V, k, first):
