@@ -143,7 +143,7 @@ __device__ __forceinline__ float readlane_f32(float v, int l) {
 constexpr int frontier_rows(int nr) { return nr >= 4 ? 6 : nr == 2 ? 3 : 2; }
 constexpr int BMAX = 64;  // entries one batch pops at most (one per lane)
 constexpr int BMIN = 3;   // candidates from which a batch is taken
-constexpr int FEW = 6;    // lists up to which several lanes share one
+constexpr int FEW = 8;    // lists up to which several lanes share one: they form at least 8 entries of it, one lane 6
 constexpr int MNT = 256;  // threads of build_mixture_kernel: wave 0 builds, the others stage and write
 // set bits of m below this lane
 __device__ __forceinline__ int lanes_below(uint64_t m) {

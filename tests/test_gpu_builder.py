@@ -293,6 +293,8 @@ def test_hf_build_mixture_contract_and_follow():
     (4, 8, 256, 256, "flat"), (8, 15, 8, 256, "flat"), (4, 9, 128, 128, "flat"), (8, 16, 64, 64, "flat"),
     (3, 7, 100, 200, "ties"), (6, 4, 33, 129, "ties"), (7, 12, 20, 65, "peaky"), (2, 3, 5, 100, "ties"),
     (8, 6, 16, 300, "shared"),   # every mode pops the same prefixes: more pops than register slots
+    (8, 16, 8, 64, "flat"), (9, 5, 12, 64, "flat"), (7, 3, 40, 100, "flat"),  # both sides of 8 lists
+    (1, 16, 64, 64, "sharp"), (8, 16, 8, 31, "sharp"), (2, 8, 3, 16, "sharp"),  # hardly a step pops more than one entry
 ])
 def test_batches_of_many_and_long_lists(K, L, k, budget, kind):
     """The batch step's two forms (lanes shared by a few lists, one lane per list) and the sequential pops between
@@ -300,7 +302,7 @@ def test_batches_of_many_and_long_lists(K, L, k, budget, kind):
     import tree_build_ext
 
     g = torch.Generator().manual_seed(K * 1000 + L * 100 + k)
-    scale = {"flat": 1.0, "ties": 1.0, "peaky": 6.0, "shared": 1.0}[kind]
+    scale = {"flat": 1.0, "ties": 1.0, "peaky": 6.0, "sharp": 20.0, "shared": 1.0}[kind]
     x = torch.randn(K, L, 4 * k + 8, generator=g) * scale
     if kind == "shared":
         x = x[:1].expand(K, -1, -1) + torch.randn(K, 1, 1, generator=g) * 1e-3
