@@ -708,7 +708,16 @@ __global__ __launch_bounds__(MNT) void build_mixture_kernel(BuildArgs a) {
     //      too little.
     bool batched = false;
     if (iter == next_check && HS > 0) {
-      batched = batch_step(f, mh, wave_min_u32(lcm));
+      // worth its enumeration only with BMIN heads below sigma, or a head (of the lanes' best ones) whose next sibling
+      // lies below it too: peaked logits fail that nearly always
+      const uint32_t sigma = wave_min_u32(lcm);
+      int heads = 0;
+#pragma unroll
+      for (int rr = 0; rr < RR; ++rr)
+        if (rr * WAVE < tail) heads += __builtin_popcountll(__builtin_amdgcn_ballot_w64(khi[rr] < sigma));
+      const uint32_t sib = key_bits(-((float)((lbw - (double)plp) + (double)plp1) + ppr));
+      const bool pair = lhi != NONE && (int)(llo & 0x3FF) + 1 < kk && sib < sigma;
+      if (heads >= BMIN || __builtin_amdgcn_ballot_w64(pair) != 0) batched = batch_step(f, mh, sigma);
       if (overflow) break;
       gap = batched ? 1 : min(2 * gap, 32);
       next_check = iter + gap;
