@@ -4,9 +4,9 @@
 //
 // The product streams the weight (vocabulary x hidden, bf16, read once per 128 drafted rows: 778 MB at a
 // 151936-token vocabulary and hidden 2560) against the drafted rows, which every workgroup shares. Three forms, by
-// the drafted rows and the vocabulary rows a CU gets (draft_head_gemm): the k-split form (few drafted rows, or a vocabulary so
-// small that one wave's walk over k would be the whole time), the wide form (more than 128 rows per CU) and, between
-// them, the pass form described here.
+// the drafted rows and the vocabulary rows a CU gets (draft_head_gemm): the k-split form (few drafted rows, or a
+// vocabulary so small that one wave's walk over k would be the whole time), the wide form (more than 128 rows per CU)
+// and, between them, the pass form described here.
 //  * The vocabulary is split evenly over the grid's workgroups (one per CU; ranges of a multiple of 8 rows),
 //    each taking its range in passes of 128 weight rows against all (up to 128) drafted rows.
 //  * Both operands stream through LDS in 64-k stages (128 weight rows and 128 drafted rows, 128 bytes each,

@@ -35,7 +35,7 @@ constexpr int PIECE = MFD_LZ_PIECE;  // log Z piece: one wave, 32 elements per l
 constexpr int PW = 16;               // waves per workgroup of kernel 1
 constexpr int NT1 = PW * 64;
 constexpr int KMAX = 256;
-constexpr int MERGE_MAX = 8192;      // accepted sizes: pieces * k (k <= 32), ceil(V / 8192) * k above
+constexpr int MERGE_MAX = 8192;      // accepted sizes (interface): pieces * k (k <= 32), ceil(V / 8192) * k above
 
 __device__ __forceinline__ float pow2i(int k) { return __uint_as_float((uint32_t)(k + 127) << 23); }
 
@@ -652,8 +652,8 @@ __device__ void row_topk(const TopkArgs& a, int row, MergeLds& ml, double* terms
   const int n = ml.n;
   if (tid == 0 && a.out_logz) a.out_logz[row] = ml.logz;
   // (For k <= 32 hundreds of candidates are a row of few groups, or one whose largest values lie close together, or
-  // ties. 8 rows, k = 8, by the bisection and so: 512 values 35 -> 11 us, 20000 falling from the first column on 35 -> 13,
-  // 151936 sorted 39 -> 16. Many equal ones are settled sooner by the bisection than by counting them against each
+  // ties. 8 rows, k = 8, by the bisection and so: 512 values 35 -> 11 us, 20000 falling from the first column on
+  // 35 -> 13, 151936 sorted 39 -> 16. Many equal ones are settled sooner by the bisection than by counting them against each
   // other: 151936 equal values 41 against 86.)
   if (n > CAND_MAX || !merge_row<NTH>(a, row, n, top + 32768, k <= 32 ? TIED_MAX : CAND_MAX, ml)) {
     auto norm = [](int key) -> int { return key == -1 ? 0 : key; };
@@ -857,7 +857,7 @@ __global__ __launch_bounds__(NTH) void topk_row_kernel(TopkArgs a) {
 
 extern "C" int64_t mfd_topk_logz_workspace_bytes(int rows, int V, int k) {
   const int64_t npieces = ((int64_t)V + PIECE - 1) / PIECE;
-  // per piece: m (4 bytes), S (8) and room for k candidate keys
+  // per piece: m (4 bytes), S (8) and 8 per rank, of which the group keys take at most 32 (the size is the interface's)
   return (int64_t)rows * npieces * (4 + 8 + 8 * (int64_t)(k > 0 ? k : 1)) + 64;
 }
 

@@ -8,8 +8,8 @@
 //     (order-preserving bits of the fp32 key, fields = mode 4b | parent 12b | depth 6b | rank 10b);
 //   - a prefix popped again by another mode reuses its node (lookup by (parent, token)); the budget
 //     counts distinct nodes.
-// The frontier, the (parent, token) -> node table and the pop records live in registers (one wave);
-// batches of pops that provably come next in the heap's order are taken in one step (see the kernel).
+// The frontier and the (parent, token) -> node table live in registers (one wave); batches of pops that provably come
+// next in the heap's order are taken in one step (see the kernel).
 // Outputs: tree[b] = tokens, depths, parents of width budget + 1 (index 0 = root: token 0, depth 0,
 // parent -1; tail entries 0, 0, -1), counts[b], and optionally the ancestor-or-self matrix anc8[b]
 // ([budget + 1]^2 int8, row i = row of parent(i) plus i; inference/hf/tree_build_ext.py:101-110).
@@ -143,7 +143,7 @@ __device__ __forceinline__ float readlane_f32(float v, int l) {
 constexpr int frontier_rows(int nr) { return nr >= 4 ? 6 : nr == 2 ? 3 : 2; }
 constexpr int BMAX = 64;  // entries one batch pops at most (one per lane)
 constexpr int BMIN = 3;   // candidates from which a batch is taken
-constexpr int FEW = 8;    // lists up to which several lanes share one: they form at least 8 entries of it, one lane 6
+constexpr int FEW = 8;    // lists up to which several lanes share one: they form 8 of its entries or more, one lane 6
 constexpr int MNT = 256;  // threads of build_mixture_kernel: wave 0 builds, the others stage and write
 // set bits of m below this lane
 __device__ __forceinline__ int lanes_below(uint64_t m) {
@@ -184,10 +184,11 @@ __device__ __forceinline__ bool pair_lt(uint32_t ka, uint32_t fa, uint32_t kb, u
 // sibling's key below its elder's: a list's candidates end before such a sibling) and after the pop that creates
 // node number budget.
 //
-// LDS layout (dynamic): slot logw f64 [cap], slot key u32 [cap], slot fields u32 [cap], slot child key
-// u32 [cap], slot last-popped rank i32 [cap] (rows >= RR always; register rows are copied in for a batch),
-// candidate logw f64 [64], (key, fields) u64 [64], slot u32 [64], records (token, lp bits) [K L k], prior f32 [16],
-// node parent / token / depth i32 [budget + 1], counter i32 [4].
+// LDS layout (dynamic): slot logw f64 [cap], candidate logw f64 [64], hash keys u64 [HS], slot key, fields, child key and
+// moved flag u32 [cap] each, hash node id and first lane i32 [HS] each, candidate (key, fields) u64 [64] and slot i32
+// [64], records (token, lp bits) [K L k], prior f32 [16], node parent / token / depth i32 [budget + 1], counter i32 [4].
+// Slots of rows >= RR live in the arrays; register rows pass through them in a batch, which is taken only while all slots
+// are register rows (so the flags beyond those are room the accepted sizes have always counted).
 // NR = register slots per lane of the node table (64 NR >= budget).
 //
 // What bounds it: the issue rate of one wave, 7-10 thousand cycles per batch step (enumeration 2.3, ranking 1-2, nodes
@@ -214,8 +215,8 @@ __global__ __launch_bounds__(MNT) void build_mixture_kernel(BuildArgs a) {
   uint32_t* fhi = reinterpret_cast<uint32_t*>(hkey + HS);
   uint32_t* flo = fhi + cap;
   uint32_t* fck = flo + cap;
-  int32_t* fmax = reinterpret_cast<int32_t*>(fck + cap);
-  int32_t* hid = fmax + cap;
+  int32_t* fmoved = reinterpret_cast<int32_t*>(fck + cap);
+  int32_t* hid = fmoved + cap;
   int32_t* hmin = hid + HS;
   uint64_t* c64 = reinterpret_cast<uint64_t*>(hmin + HS);  // a batch's candidates: key in the upper, fields in the lower half
   int32_t* cs = reinterpret_cast<int32_t*>(c64 + BMAX);
@@ -231,7 +232,7 @@ __global__ __launch_bounds__(MNT) void build_mixture_kernel(BuildArgs a) {
     stage_records<MNT>(lpb, static_cast<const int64_t*>(a.ids) + (int64_t)b * nlp, rec, nlp, (int)threadIdx.x);
   else
     stage_records<MNT>(lpb, static_cast<const int32_t*>(a.ids) + (int64_t)b * nlp, rec, nlp, (int)threadIdx.x);
-  for (int s = threadIdx.x; s < cap; s += MNT) fmax[s] = -1;
+  for (int s = threadIdx.x; s < cap; s += MNT) fmoved[s] = -1;
   for (int h = threadIdx.x; h < HS; h += MNT) {
     hkey[h] = HEMPTY;
     hid[h] = -1;
@@ -338,8 +339,9 @@ __global__ __launch_bounds__(MNT) void build_mixture_kernel(BuildArgs a) {
 
   int count = 0, tail = K, alive = K, hashed = 0, next_check = 0, gap = 1;
   bool overflow = false;
-  // Batch step: pops the prefix of the frontier order below sigma at once (see above). Returns false, with
-  // nothing changed, when fewer than BMIN entries are certain or more than 64 lists qualify.
+  // Batch step: pops the prefix of the frontier order below sigma (lowered where more than 64 lists or entries lie below
+  // it) at once (see above). Returns false, with nothing changed, when fewer than BMIN entries are certain, when the
+  // frontier reaches beyond the registers, or when more than 64 heads share the smallest key.
   auto batch_step = [&](uint32_t f1, uint32_t mh, uint32_t sigma) -> bool {
     if (tail > RR * WAVE) return false;
     // more than 64 lists below sigma: a lower one
@@ -644,7 +646,7 @@ __global__ __launch_bounds__(MNT) void build_mixture_kernel(BuildArgs a) {
     // lists in new slots
     const bool last = live && enext >= nb;
     if (last) {
-      fmax[eslot] = -2;  // moved
+      fmoved[eslot] = -2;  // moved
       if (has_next) {
         fhi[eslot] = nkey;
         flo[eslot] = nfld;
@@ -680,13 +682,13 @@ __global__ __launch_bounds__(MNT) void build_mixture_kernel(BuildArgs a) {
     for (int rr = 0; rr < RR; ++rr) {
       if (rr * WAVE >= tail) continue;
       const int s = rr * WAVE + lane;
-      if ((ql[rr] && fmax[s] == -2) || (s >= told && s < tail)) {
+      if ((ql[rr] && fmoved[s] == -2) || (s >= told && s < tail)) {
         khi[rr] = fhi[s];
         klo[rr] = flo[s];
         kck[rr] = fck[s];
         klw[rr] = flogw[s];
       }
-      if (ql[rr]) fmax[s] = -1;
+      if (ql[rr]) fmoved[s] = -1;
     }
     rescan(tail);
     prefetch();

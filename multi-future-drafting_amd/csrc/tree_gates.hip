@@ -36,11 +36,12 @@ __device__ __forceinline__ float softplus_torch(float x) { return x > 20.f ? x :
 
 // What bounds it: latency, that of two trips to memory (offsets, then parents and projections) and of the chain of a
 // few hundred dependent operations of softplus and sigmoid, which the two waves per SIMD of a CU's one workgroup do not
-// hide: so the softplus is formed once per (node, head), by all threads at once. 8 trees of 128 nodes, 32 heads: 5.5 us;
-// 11 us with g formed again for every descendant, 16.8 us for threads that walked in memory, once per summed ancestor.
+// hide: so the softplus is formed once per (node, head), by all threads at once. 8 trees of 128 nodes, 32 heads:
+// 5.5 us; 11 us with g formed again for every descendant, 16.8 us for threads that walked in memory, once per summed
+// ancestor.
 constexpr int NT = 512;
 constexpr int HB = 4;       // heads per workgroup: 64 workgroups for 8 requests of 32 heads
-constexpr int NMAX = 1024;  // nodes of a request held in LDS; a larger request's nodes go to workgroups that walk in memory
+constexpr int NMAX = 1024;  // nodes of a request held in LDS; those of a larger one go to workgroups that walk in memory
 constexpr int NB = NT / HB; // nodes of such a workgroup
 constexpr int PATH = 16;    // path entries held in LDS; deeper nodes walk again per ancestor
 
@@ -93,8 +94,8 @@ __device__ void walk_in_memory(const GatesArgs& a, int node, int h) {
 }
 
 // Workgroups 0 .. R hblocks - 1: one per request of at most NMAX nodes and four heads. Then, in batches that can hold a
-// larger request, one per NB nodes of the batch and four heads for the nodes of such requests: 1400 nodes, 32 heads take
-// 88 of them (15 us; 144 us by the eight workgroups of the request and its heads).
+// larger request, one per NB nodes of the batch and four heads for the nodes of such requests: 1400 nodes, 32 heads
+// take 88 of them (15 us; 144 us by the eight workgroups of the request and its heads).
 __global__ __launch_bounds__(NT) void tree_gates_kernel(GatesArgs a) {
   __shared__ float sp[NMAX][HB];  // softplus of every (node, head)
   __shared__ int16_t par[NMAX], depth[NMAX];

@@ -377,11 +377,12 @@ constexpr int LT = 512;  // threads of the main kernel: one per node in phase T
 // TWO: two workgroups per CU, for grids of more than one round and trees of at most TWO_NODES nodes. The phases wait on
 // memory, on the serial chain of T and on the stores in turn (VALU 45 % busy, waves waiting 53 % of their time), and one
 // resident workgroup leaves the CU idle meanwhile. So half the LDS (large_lds) and at most 128 registers: the S0
-// fragments are read after T, and tiles are requested one ahead and after T. 4 x 257 nodes, H 32: 35.8 -> 33.0 us;
+// fragments are read after T, and tiles are requested one ahead and after T. 4 x 257 nodes, H 32: 32.6 -> 28.7 us;
 // two layers with the context, 8 x 130: 97.4 -> 86.8, one 257-node tree with H 48 (16 columns): 71.0 -> 59.8.
 // Longer trees keep one workgroup per CU.
 template <int NMAX, int CT, bool ONE, bool TWO>
-__global__ __launch_bounds__(LT) __attribute__((amdgpu_waves_per_eu(TWO ? 4 : 2))) void tree_gdn_large_kernel(GdnLargeArgs a, int nml) {
+__global__ __launch_bounds__(LT) __attribute__((amdgpu_waves_per_eu(TWO ? 4 : 2))) void tree_gdn_large_kernel(GdnLargeArgs a,
+                                                                                                            int nml) {
   constexpr int CW = 16 * CT;                 // value columns of a workgroup
   constexpr int MAXT = ((TWO && NMAX > TWO_NODES ? TWO_NODES : NMAX) / 16 + 7) / 8;  // 16-node tiles per wave at most
   extern __shared__ __align__(16) uint8_t lds[];
@@ -550,16 +551,17 @@ __global__ __launch_bounds__(LT) __attribute__((amdgpu_waves_per_eu(TWO ? 4 : 2)
   bf16x8 sb[CT][D / 32];
   auto read_s0 = [&]() __attribute__((always_inline)) {
 #pragma unroll
-  for (int ct = 0; ct < CT; ++ct)
+    for (int ct = 0; ct < CT; ++ct)
 #pragma unroll
-    for (int kc = 0; kc < D / 32; ++kc) {
-      const float* src = S0L + (32 * kc + 8 * g4) * SS + 16 * ct + l16;
-      u32x4 pk;
+      for (int kc = 0; kc < D / 32; ++kc) {
+        const float* src = S0L + (32 * kc + 8 * g4) * SS + 16 * ct + l16;
+        u32x4 pk;
 #pragma unroll
-      for (int e = 0; e < 4; ++e)
-        pk[e] = __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2){src[(2 * e) * SS], src[(2 * e + 1) * SS]}, bf16x2));
-      sb[ct][kc] = __builtin_bit_cast(bf16x8, pk);
-    }
+        for (int e = 0; e < 4; ++e)
+          pk[e] = __builtin_bit_cast(
+              uint32_t, __builtin_convertvector((f32x2){src[(2 * e) * SS], src[(2 * e + 1) * SS]}, bf16x2));
+        sb[ct][kc] = __builtin_bit_cast(bf16x8, pk);
+      }
   };
   if constexpr (!TWO) read_s0();
 
@@ -630,9 +632,9 @@ __global__ __launch_bounds__(LT) __attribute__((amdgpu_waves_per_eu(TWO ? 4 : 2)
     }
     *reinterpret_cast<f32x4*>(&KQ[i * 2 * MAXD + 4 * c]) = xv;
   }
-  // (one workgroup per CU) the first tiles' K / Q rows and v, in flight during T: waves 0-3 (the T threads of the first 256 nodes) request
-  // theirs before the barrier, the others after it, where their issue (a wave waits there for room in the CU's
-  // load queue) runs beside T instead of holding the barrier
+  // (one workgroup per CU) the first tiles' K / Q rows and v, in flight during T: waves 0-3 (the T threads of the first
+  // 256 nodes) request theirs before the barrier, the others after it, where their issue (a wave waits there for room in
+  // the CU's load queue) runs beside T instead of holding the barrier
   if (!TWO && w < 4) {
 #pragma unroll
     for (int j = 0; j < PRE; ++j) load_tile(w + 8 * j, j);

@@ -25,8 +25,8 @@ def topk_logz(logits: torch.Tensor, k: int, ids_dtype=torch.int64, with_logz: bo
     log Z [R] or None) buffers to write into; ``workspace``: a uint8 buffer of at least
     mfd_topk_logz_workspace_bytes(R, V, k) bytes (both optional, for graph capture without allocation).
     Limits: k <= 256; for bf16 ceil(V / 2048) * max(k, 1) <= 8192 for k <= 32 and ceil(V / 8192) * k <= 8192
-    above; larger requests raise MFDError. fp16 / fp32 logits (the reference
-    takes any float dtype) go through a kernel of their own with an fp32 log Z (no workspace, no V limit)."""
+    above; larger requests raise MFDError. fp16 / fp32 logits (the reference takes any float dtype) go through a
+    kernel of their own with an fp32 log Z (no workspace, no V limit)."""
     mfd_hip.require_cuda(logits, vocab_ids)
     wide = {torch.float32: 0, torch.float16: 1}.get(logits.dtype)  # MFD_DTYPE_F32 / MFD_DTYPE_F16
     if logits.dtype != torch.bfloat16 and wide is None:

@@ -516,8 +516,8 @@ def test_draft_head_gemm_forms(M, N, K):
 
 def test_draft_head_gemm_full_vocabulary_sampled():
     """The config-1 draft head shape: 8 modes x 15 drafted rows, hidden 2560, the full 151936-token vocabulary
-    (every workgroup takes several 128-row passes; the last pass of each is partial). 4096 sampled columns
-    against the exact product, every logit finite, the row padding untouched."""
+    (the wide form, 594 rows per workgroup, the last tile of each partial). 4096 sampled columns against the exact
+    product, every logit finite, the row padding untouched."""
     import mfd_hip
 
     print("case: draft head gemm M=120 N=151936 K=2560 (sampled)", flush=True)
